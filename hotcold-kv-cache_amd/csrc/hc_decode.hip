@@ -183,61 +183,128 @@ __global__ __launch_bounds__(256) void h2o_evict_one_kernel(const float* scores,
 
 // Per-token eviction score of the reference kernel (kernels.py:66-67, 134-136):
 //   loss[b,s] = dtype( mean_h( p[b,h,s] / l[b,h] * mean_d |v[b,hk(h),s,d]| ) )
-// with p = exp(logit - max) (the max cancels), and evict_idx[b] = first argmin.
+// with p = exp(logit - max) (the max cancels), and evict_idx[b] = first argmin
+// (NaN lowest, as torch.argmin ranks it).
+//
+// Bound by reading V once more.  grid (cdiv(S, kEvKeys), B), block 256: a
+// workgroup owns kEvKeys keys, and its threads take (key, KV head) pairs, so
+// every V row is one thread's, which sums |v| in dimension order.  A wave
+// loads its 64 rows in whole 128-byte lines (8 lanes a row) and hands them to
+// their threads through LDS: with each thread loading its own row the lines
+// fell out of the first cache between their eight 16-byte loads (25 us).  Then
+// one thread per key runs the chain over the query heads, KV heads in order.
+// A batch row's minimum is an atomic on (loss key, key index), and its last
+// workgroup to finish writes the index (decode_attn_kernel resets both words).
+// One workgroup per batch row, each thread walking the V rows element by
+// element, took 2519 us at 4 x 4099 keys, 8 KV heads of 128 in bf16; this form
+// 19 us.
+constexpr int kEvKeys = 32;
+constexpr int kEvHeads = 8;      // KV heads per pass
+constexpr int kEvMaxG = 16;      // query heads per KV head (decode's limit)
+constexpr int kEvPre = 4;        // ... whose logits are loaded ahead of the V rows
+constexpr int kEvCols = 2;       // 128-byte columns of the rows in flight
+
 template <typename T>
 __global__ __launch_bounds__(256) void evict_score_kernel(const float* scores, const float* ml,
                                                           const T* v, int64_t v_sb, int64_t v_sh,
-                                                          int64_t v_ss, int Hq, int G, int S, int D,
-                                                          float* loss, int64_t* idx) {
-  const int b = blockIdx.x;
-  float best = INFINITY;
-  int best_i = 0x7fffffff;
-  for (int s = threadIdx.x; s < S; s += blockDim.x) {
-    float tot = 0.f;
-    for (int hk = 0; hk < Hq / G; ++hk) {
-      const T* vr = v + b * v_sb + hk * v_sh + (int64_t)s * v_ss;
-      float av = 0.f;
-      for (int d = 0; d < D; ++d) av += fabsf(to_f32(vr[d]));
-      av /= (float)D;
-      for (int g = 0; g < G; ++g) {
-        const int h = hk * G + g;
-        const float M = ml[((int64_t)b * Hq + h) * 2 + 0];
-        const float L = ml[((int64_t)b * Hq + h) * 2 + 1];
-        const float sc = scores[((int64_t)b * Hq + h) * S + s];
-        const float pn = (sc == -INFINITY) ? 0.f : exp2f(sc - M) / L;
-        tot += pn * av;
+                                                          int64_t v_ss, int Hk, int G, int S, int D,
+                                                          float* loss, int64_t* idx, unsigned long long* vmin) {
+  static_assert(kEvKeys * kEvHeads == 256, "one (key, KV head) pair per thread");
+  constexpr int kPer = 16 / (int)sizeof(T);    // elements per 16-byte piece
+  __shared__ u32x4 sm_v[4][64][8];             // a wave's rows, one column; piece p of row r at p ^ (r & 7)
+  __shared__ float sm_p[kEvMaxG][kEvHeads][kEvKeys];
+  __shared__ float sm_av[kEvHeads][kEvKeys];
+  const int b = blockIdx.y, tid = threadIdx.x, kl = tid % kEvKeys, hl = tid / kEvKeys;
+  const int lane = tid & 63, wave = tid >> 6;
+  const int s = blockIdx.x * kEvKeys + kl;
+  const int Hq = Hk * G;
+  float tot = 0.f;
+  for (int h0 = 0; h0 < Hk; h0 += kEvHeads) {
+    const int hk = h0 + hl;
+    const int64_t hq = (int64_t)b * Hq + min(hk, Hk - 1) * G;
+    const int sc_s = min(s, S - 1);
+    float sc[kEvPre], M[kEvPre], L[kEvPre];   // in flight with the V rows
+#pragma unroll
+    for (int g = 0; g < kEvPre; ++g) {
+      const int64_t h = hq + min(g, G - 1);
+      sc[g] = scores[h * S + sc_s];
+      M[g] = ml[h * 2 + 0];
+      L[g] = ml[h * 2 + 1];
+    }
+    // row 8 i + lane / 8 of the wave's 64, piece lane % 8 of each column;
+    // rows and pieces past the end repeat the last one (not summed)
+    const T* vr[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int r = 64 * wave + 8 * i + (lane >> 3);
+      vr[i] = v + b * v_sb + min(h0 + r / kEvKeys, Hk - 1) * v_sh +
+              (int64_t)min((int)blockIdx.x * kEvKeys + r % kEvKeys, S - 1) * v_ss;
+    }
+    float av = 0.f;
+    for (int d0 = 0; d0 < D; d0 += kEvCols * 8 * kPer) {
+      u32x4 x[kEvCols][8];
+#pragma unroll
+      for (int c = 0; c < kEvCols; ++c)
+#pragma unroll
+        for (int i = 0; i < 8; ++i) x[c][i] = ld16(vr[i] + min(d0 + (c * 8 + (lane & 7)) * kPer, D - kPer));
+#pragma unroll
+      for (int c = 0; c < kEvCols; ++c) {
+        if (d0 + c * 8 * kPer >= D) break;     // uniform
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < 8; ++i) sm_v[wave][8 * i + (lane >> 3)][(lane & 7) ^ (lane >> 3)] = x[c][i];
+        __syncthreads();
+#pragma unroll
+        for (int p = 0; p < 8; ++p)
+          if (d0 + (c * 8 + p) * kPer < D) {
+            const u32x4 y = sm_v[wave][lane][p ^ (lane & 7)];
+            const uint32_t w[4] = {y[0], y[1], y[2], y[3]};
+#pragma unroll
+            for (int i = 0; i < kPer; ++i) av += fabsf(Unpack<T>::get(w, i));
+          }
       }
     }
-    const float lv = to_f32(from_f32<T>(tot / (float)Hq));
-    loss[(int64_t)b * S + s] = lv;
-    if (lv < best || (lv != lv && best == best)) {  // NaN ranks lowest (torch.argmin)
-      best = lv;
-      best_i = s;
-    }
-  }
-  __shared__ float sb[256];
-  __shared__ int si[256];
-  sb[threadIdx.x] = best;
-  si[threadIdx.x] = best_i;
-  __syncthreads();
-  for (int o = 128; o > 0; o >>= 1) {
-    if ((int)threadIdx.x < o) {
-      const float x = sb[threadIdx.x + o];
-      const int xi = si[threadIdx.x + o];
-      const float y = sb[threadIdx.x];
-      const int yi = si[threadIdx.x];
-      const bool xnan = (x != x), ynan = (y != y);
-      bool take;
-      if (xnan || ynan) take = xnan && (!ynan || xi < yi);
-      else take = (x < y) || (x == y && xi < yi);
-      if (take) {
-        sb[threadIdx.x] = x;
-        si[threadIdx.x] = xi;
-      }
+    sm_av[hl][kl] = av / (float)D;
+#pragma unroll
+    for (int g = 0; g < kEvPre; ++g)
+      if (g < G) sm_p[g][hl][kl] = (sc[g] == -INFINITY) ? 0.f : exp2f(sc[g] - M[g]) / L[g];
+    for (int g = kEvPre; g < G; ++g) {
+      const float sg = scores[(hq + g) * S + sc_s];
+      sm_p[g][hl][kl] = (sg == -INFINITY) ? 0.f : exp2f(sg - ml[(hq + g) * 2]) / ml[(hq + g) * 2 + 1];
     }
     __syncthreads();
+    if (tid < kEvKeys && s < S)
+      for (int i = 0; i < min(kEvHeads, Hk - h0); ++i) {
+        const float av = sm_av[i][tid];
+        float p[kEvPre];
+#pragma unroll
+        for (int g = 0; g < kEvPre; ++g) p[g] = sm_p[min(g, G - 1)][i][tid];
+#pragma unroll
+        for (int g = 0; g < kEvPre; ++g) tot = g < G ? tot + p[g] * av : tot;
+        for (int g = kEvPre; g < G; ++g) tot += sm_p[g][i][tid] * av;
+      }
+    __syncthreads();
   }
-  if (threadIdx.x == 0) idx[b] = si[0];
+  if (tid >= 64) return;
+  uint64_t best = ~0ull;
+  if (tid < kEvKeys && s < S) {
+    const float lv = to_f32(from_f32<T>(tot / (float)Hq));
+    loss[(int64_t)b * S + s] = lv;
+    best = ((uint64_t)(lv != lv ? 0u : order_key(lv)) << 32) | (uint32_t)s;
+  }
+#pragma unroll
+  for (int o = kEvKeys / 2; o > 0; o >>= 1) {
+    const uint64_t x = ((uint64_t)__shfl_xor((uint32_t)(best >> 32), o, 64) << 32) | __shfl_xor((uint32_t)best, o, 64);
+    best = x < best ? x : best;
+  }
+  if (tid == 0) {
+    // the minimum's returned value is waited for, so it is in place before the
+    // count rises; nothing else crosses workgroups, so no fence is needed
+    const unsigned long long was = atomicMin(vmin + 2 * b, (unsigned long long)best);
+    __asm__ volatile("" ::"v"(was) : "memory");
+    if (atomicAdd(vmin + 2 * b + 1, 1ull) + 1 == gridDim.x)
+      idx[b] = (int64_t)(uint32_t)atomicMin(vmin + 2 * b, ~0ull);
+  }
 }
 
 // The first kCounterBytes of a decode workspace hold the in-kernel merge's
@@ -334,10 +401,10 @@ static DecodeShape decode_call_shape(int es, int64_t B, int64_t Hq, int64_t Hk, 
 }
 
 struct DecodeLayout {
-  int64_t part_off, scores_off, ml_off, total;
+  int64_t part_off, scores_off, ml_off, min_off, total;
 };
 
-// [counters (kCounterBytes)][split partials][eviction logits][(max, sum)]
+// [counters (kCounterBytes)][split partials][eviction logits][(max, sum)][row minima]
 static DecodeLayout decode_layout(int64_t B, int64_t Hq, int64_t Hk, int64_t D, int64_t S,
                                   int64_t splits, int with_evict) {
   DecodeLayout L;
@@ -349,7 +416,8 @@ static DecodeLayout decode_layout(int64_t B, int64_t Hq, int64_t Hk, int64_t D, 
   const int64_t scores_bytes = with_evict ? B * Hq * S * 4 : 0;
   L.ml_off = align256(L.scores_off + scores_bytes);
   const int64_t ml_bytes = with_evict ? B * Hq * 2 * 4 : 0;
-  L.total = align256(L.ml_off + ml_bytes);
+  L.min_off = align256(L.ml_off + ml_bytes);
+  L.total = align256(L.min_off + (with_evict ? B * 16 : 0));
   return L;
 }
 
@@ -452,6 +520,7 @@ static int decode_impl(int dtype, int64_t B, int64_t Hq, int64_t Hk, int64_t D, 
   a.part = reinterpret_cast<float*>(ws + lay.part_off);
   a.scores = with_evict ? reinterpret_cast<float*>(ws + lay.scores_off) : nullptr;
   a.ml = with_evict ? reinterpret_cast<float*>(ws + lay.ml_off) : nullptr;
+  a.evict_min = evict_loss ? reinterpret_cast<unsigned long long*>(ws + lay.min_off) : nullptr;
   a.B = (int)B; a.Hq = (int)Hq; a.Hk = (int)Hk; a.G = G; a.S = (int)S;
   a.splits = splits;
   a.keys_per_split = (int)shape.kps;
@@ -501,15 +570,14 @@ static int decode_impl(int dtype, int64_t B, int64_t Hq, int64_t Hk, int64_t D, 
                        h2o_sb, h2o_sh);
     if ((rc = check_launch("h2o_accum")) != HC_OK) return rc;
   } else if (with_evict) {
-    if (dtype == HC_DTYPE_F16)
-      hipLaunchKernelGGL(evict_score_kernel<half_t>, dim3((unsigned)B), dim3(256), 0, st, a.scores, a.ml,
-                         (const half_t*)v, v_sb, v_sh, v_ss, (int)Hq, G, (int)S, (int)D, evict_loss, evict_idx);
-    else if (dtype == HC_DTYPE_BF16)
-      hipLaunchKernelGGL(evict_score_kernel<bf16_t>, dim3((unsigned)B), dim3(256), 0, st, a.scores, a.ml,
-                         (const bf16_t*)v, v_sb, v_sh, v_ss, (int)Hq, G, (int)S, (int)D, evict_loss, evict_idx);
-    else
-      hipLaunchKernelGGL(evict_score_kernel<float>, dim3((unsigned)B), dim3(256), 0, st, a.scores, a.ml,
-                         (const float*)v, v_sb, v_sh, v_ss, (int)Hq, G, (int)S, (int)D, evict_loss, evict_idx);
+    const dim3 grid((unsigned)cdiv(S, kEvKeys), (unsigned)B);
+    auto launch = [&](auto kern, auto vp) {
+      hipLaunchKernelGGL(kern, grid, dim3(256), 0, st, a.scores, a.ml, vp, v_sb, v_sh, v_ss, (int)Hk, G, (int)S,
+                         (int)D, evict_loss, evict_idx, a.evict_min);
+    };
+    if (dtype == HC_DTYPE_F16) launch(evict_score_kernel<half_t>, (const half_t*)v);
+    else if (dtype == HC_DTYPE_BF16) launch(evict_score_kernel<bf16_t>, (const bf16_t*)v);
+    else launch(evict_score_kernel<float>, (const float*)v);
     if ((rc = check_launch("evict_score")) != HC_OK) return rc;
   }
   return HC_OK;

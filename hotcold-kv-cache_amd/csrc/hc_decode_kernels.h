@@ -105,6 +105,9 @@ struct DecodeArgs {
   // previous launch (epoch itself if not known).
   unsigned long long* counters;
   uint32_t epoch, prev_epoch;
+  // Eviction score: per batch row its running minimum and its count of
+  // finished workgroups (evict_score_kernel), reset by this launch.
+  unsigned long long* evict_min;
 };
 static_assert(offsetof(DecodeArgs, Hq) + sizeof(int) <= 128, "the first loads' fields must fit bytes 0-127");
 static_assert(offsetof(DecodeArgs, B) == 128 && offsetof(DecodeArgs, cur_pos) + sizeof(void*) <= 256,
@@ -639,6 +642,12 @@ __global__ __launch_bounds__(64 * NW, MINW) void decode_attn_kernel(DecodeArgs a
   const uint32_t k_rowb = (uint32_t)(a.k_ss * (int64_t)sizeof(T));
   const uint32_t v_rowb = (uint32_t)(a.v_ss * (int64_t)sizeof(T));
 
+  if constexpr (EVICT && !APPEND) {
+    if (a.evict_min && split == 0 && hk == 0 && threadIdx.x == 0) {
+      a.evict_min[2 * b] = ~0ull;
+      a.evict_min[2 * b + 1] = 0ull;
+    }
+  }
 
   constexpr bool MX = sizeof(T) == 2;
   typename DecodeState<T, D, GM>::type st;

@@ -319,6 +319,35 @@ def test_decode_strided_views_and_evict_score():
         assert want_loss[b, int(idx[b])] <= want_loss[b].min() * (1 + 2e-3) + 1e-7
 
 
+@pytest.mark.parametrize("B,Hq,Hk,S,D,dtype,masked", [
+    (1, 4, 4, 1, 16, torch.float16, False),           # one key, one KV pass with heads left over
+    (3, 32, 8, 31, 128, torch.float16, True),         # under one workgroup's keys
+    (2, 32, 8, 33, 128, torch.bfloat16, False),       # one key in the last workgroup
+    (2, 24, 12, 257, 64, torch.float16, True),        # two passes over the KV heads, the second partial
+    (2, 32, 2, 1000, 128, torch.bfloat16, True),      # the largest group
+    (2, 8, 2, 130, 256, torch.float32, False),        # rows of several load batches
+    (4, 32, 8, 4099, 128, torch.bfloat16, True),
+])
+def test_evict_score_and_its_first_minimum(B, Hq, Hk, S, D, dtype, masked):
+    q, k, v = _randn((B, Hq, 1, D), 21, dtype), _randn((B, Hk, S, D), 22, dtype), _randn((B, Hk, S, D), 23, dtype)
+    mask = (torch.rand((B, S), generator=torch.Generator().manual_seed(24)) < 0.8) if masked else None
+    if masked:
+        mask[:, S - 1] = True
+    dm = mask.to(DEV) if masked else None
+    want, _ = ref.evict_scores(q, k, v, 0.088, mask)
+    # the loss is rounded once to dtype (half an ulp); its fp32 terms (a logit of magnitude up to about 6 in the
+    # exponent, D + Hq additions) are below 2e-5 of it
+    rtol = {torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8, torch.float32: 0.0}[dtype] + 2e-5
+    for _ in range(2):                                # the second launch finds the workspace as the first left it
+        _, loss, idx = ops.decode_attention(q.to(DEV), k.to(DEV), v.to(DEV), 0.088, mask=dm, with_evict=True)
+        got = loss.cpu().numpy()
+        assert np.allclose(got, want, rtol=rtol, atol=6e-8)    # fp16's smallest step
+        assert np.array_equal(idx.cpu().numpy(), got.argmin(axis=1))
+    v[0, :, S // 2, 0] = float("nan")                 # a NaN loss ranks lowest
+    _, loss, idx = ops.decode_attention(q.to(DEV), k.to(DEV), v.to(DEV), 0.088, mask=dm, with_evict=True)
+    assert torch.isnan(loss[0, S // 2]) and int(idx[0]) == S // 2
+
+
 APPEND_CASES = [
     # B, Hq, Hk, cap, n (cached rows), D, dtype, splits
     (1, 32, 8, 700, 573, 128, torch.float16, 0),    # 8k/budget-512 hot buffer, mid-decode
