@@ -20,9 +20,26 @@
 // Kernels (one stream, in order):
 //   qmean   -> qf (fp64 [B][Hk][Wpad][D], rows >= W zeroed)
 //   logits  -> L (fp32 [B][Hk][W][S]) + row max (atomicMax on order keys)
+//              (both in the int8-digit form of hc_logits_i8.h for 2-byte keys
+//              of head dim 64 or 128 and groups of 2^n query heads)
 //   rowsum  -> l_w (uint64, 64-bit atomics)            [SNAPKV only]
 //   imp     -> pooled fp32 scores [B][Hk][S]
 #include "hc_common.h"
+
+namespace hc {
+
+constexpr int kNeverRead = 512;  // > the 256 (rowsum) and 270 (imp_pool) read margins
+
+// Per window row, for the importance pass: the row max and 1/l_w in fp64.
+// Rows are padded to a multiple of kStatPad per (b, h); the padding rows hold
+// {+inf, 0}, so they add an exact zero to the importance chain.
+struct RowStat {
+  double m, inv;
+};
+constexpr int kStatPad = 16;
+
+}  // namespace hc
+#include "hc_logits_i8.h"
 
 namespace hc {
 
@@ -38,16 +55,8 @@ static int64_t row_block(int64_t W) { return W > kRowBlk ? kRowBlkWide : kRowBlk
 constexpr int kMaxPool = 32;  // max half-width of the pooling window
 
 struct ScoreLayout {
-  int64_t wpad, nchunk_m, qf_off, logits_off, rmax_off, rstat_off, total;
+  int64_t wpad, nchunk_m, qf_off, logits_off, rmax_off, rstat_off, qd_off, qrow_off, total;
 };
-
-// Per window row, for the importance pass: the row max and 1/l_w in fp64.
-// Rows are padded to a multiple of kStatPad per (b, h); the padding rows hold
-// {+inf, 0}, so they add an exact zero to the importance chain.
-struct RowStat {
-  double m, inv;
-};
-constexpr int kStatPad = 16;
 
 static int64_t al256(int64_t x) { return (x + 255) & ~(int64_t)255; }
 
@@ -59,7 +68,9 @@ static ScoreLayout score_layout(int64_t B, int64_t Hk, int64_t S, int64_t D, int
   L.logits_off = al256(L.qf_off + B * Hk * L.wpad * D * 8);
   L.rmax_off = al256(L.logits_off + B * Hk * W * S * 4);
   L.rstat_off = al256(L.rmax_off + B * Hk * W * 4);
-  L.total = al256(L.rstat_off + B * Hk * cdiv(W, kStatPad) * kStatPad * (int64_t)sizeof(RowStat));
+  L.qd_off = al256(L.rstat_off + B * Hk * cdiv(W, kStatPad) * kStatPad * (int64_t)sizeof(RowStat));
+  L.qrow_off = al256(L.qd_off + B * Hk * L.wpad * D * kDigits);
+  L.total = al256(L.qrow_off + B * Hk * L.wpad * (int64_t)sizeof(QDigitRow));
   return L;
 }
 
@@ -177,7 +188,6 @@ struct KOperand<float> {
 // 16 at the 8k, 32-layer batch (one round of 1024 workgroups), 1 for one
 // 8k layer.
 constexpr int kLogitChunks = 16;
-constexpr int kNeverRead = 512;  // > the 256 (rowsum) and 270 (imp_pool) read margins
 constexpr int kLogitTargetWg = 1024;
 constexpr int kKRing = 4;
 
@@ -644,6 +654,37 @@ __global__ void head_mean_kernel(const float* __restrict__ x, int H, int S, floa
   out[(int64_t)b * S + s] = (float)(acc / (double)H);
 }
 
+// The int8 kernel's workgroups at their fewest chunks: five per CU.
+constexpr int kDigitTargetWg = 1280;
+
+template <typename T>
+static void launch_logits_i8(int mode, int64_t B, int64_t Hk, int64_t S, int64_t D, int64_t W,
+                             int64_t wpad, const T* k, const T* const* k_rows, int64_t k_sb, int64_t k_sh,
+                             int64_t k_ss, uint32_t k_bytes, const double* qf, const int8_t* qd,
+                             const QDigitRow* qrow, double scal, float* logits, uint32_t* rmax, hipStream_t st) {
+  const int rows = W > 32 ? 64 : (W > 16 ? 32 : 16);     // wpad is a multiple of each
+  const int64_t nrb = cdiv(W, rows), wg1 = cdiv(S, (int64_t)kDigitChunk) * Hk * nrb * B;
+  const int cpw = (int)std::max<int64_t>(1, std::min<int64_t>(kLogitChunks, wg1 / kDigitTargetWg));
+  const dim3 grid((unsigned)cdiv(S, (int64_t)kDigitChunk * cpw), (unsigned)(Hk * nrb), (unsigned)B);
+  auto launch = [&](auto kern) {
+    hipLaunchKernelGGL(kern, grid, dim3(256), 0, st, k, k_rows, k_sb, k_sh, k_ss, k_bytes, qf, qd, qrow, (int)Hk,
+                       (int)S, (int)W, (int)wpad, scal, cpw, (int)S, logits, rmax);
+  };
+  auto pick = [&](auto dim) {
+    constexpr int DC = decltype(dim)::value;
+    auto by_rows = [&](auto mode_c) {
+      constexpr int M = decltype(mode_c)::value;
+      if (rows == 16) launch(logits_i8_kernel<T, M, DC, 1>);
+      else if (rows == 32) launch(logits_i8_kernel<T, M, DC, 2>);
+      else launch(logits_i8_kernel<T, M, DC, 4>);
+    };
+    if (mode == HC_SCORE_SNAPKV) by_rows(std::integral_constant<int, HC_SCORE_SNAPKV>{});
+    else by_rows(std::integral_constant<int, HC_SCORE_RAWSUM>{});
+  };
+  if (D == 128) pick(std::integral_constant<int, 128>{});
+  else pick(std::integral_constant<int, 64>{});
+}
+
 template <typename T>
 static void launch_score(const ScoreLayout& lay, char* ws, int mode, int64_t B, int64_t Hq, int64_t Hk, int64_t S,
                          int64_t D, int64_t W, const void* q, const void* const* q_rows, int64_t q_sb, int64_t q_sh,
@@ -656,36 +697,60 @@ static void launch_score(const ScoreLayout& lay, char* ws, int mode, int64_t B, 
   RowStat* rstat = reinterpret_cast<RowStat*>(ws + lay.rstat_off);
   const int rows = (int)row_block(W);
   const int nrb = (int)(lay.wpad / rows);
-  hipLaunchKernelGGL(qmean_kernel<T>, dim3((unsigned)lay.wpad, (unsigned)Hk, (unsigned)B),
-                     dim3((unsigned)(D < 64 ? 64 : D)), 0, st, (const T*)q, (const T* const*)q_rows, q_sb, q_sh,
-                     q_ss, q_row0, (int)Hq,
-                     (int)Hk, (int)W, (int)lay.wpad, (int)D, qf, rmax, rstat);
-  const size_t lds = (size_t)(rows * (D + 1) * 8);
+  int8_t* qd = reinterpret_cast<int8_t*>(ws + lay.qd_off);
+  QDigitRow* qrow = reinterpret_cast<QDigitRow*>(ws + lay.qrow_off);
+  // The int8 digits serve 2-byte keys of the compiled head dims.  A group
+  // whose size is not a power of two has means that no fixed point holds, so
+  // most of its tiles would be redone in fp64.
+  const int64_t G = Hq % Hk == 0 ? Hq / Hk : Hq;
+  const bool dig = sizeof(T) == 2 && (D == 64 || D == 128) && (G & (G - 1)) == 0;
   const uint32_t k_bytes = (uint32_t)(((S - 1) * k_ss + D) * (int64_t)sizeof(T));
-  const int64_t wg1 = cdiv(S, (int64_t)kChunkM) * Hk * nrb * B;  // workgroups at one chunk each
-  const int cpw = (int)std::max<int64_t>(1, std::min<int64_t>(kLogitChunks, wg1 / kLogitTargetWg));
-  const dim3 grid((unsigned)cdiv(S, (int64_t)kChunkM * cpw), (unsigned)(Hk * nrb), (unsigned)B);
-  auto launch = [&](auto kern) {
-    if (lds > 48 * 1024)
-      (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    hipLaunchKernelGGL(kern, grid, dim3(256), lds, st, (const T*)k, (const T* const*)k_rows, k_sb, k_sh, k_ss,
-                       k_bytes, (const double*)qf,
-                       (int)Hk, (int)S, (int)D, (int)W, (int)lay.wpad, scal, cpw, logits, rmax);
-  };
-  if (mode == HC_SCORE_SNAPKV) {
-    if (rows == kRowBlk) {
-      if (D == 128) launch(logits_kernel<T, HC_SCORE_SNAPKV, 128, 2>);
-      else if (D == 64) launch(logits_kernel<T, HC_SCORE_SNAPKV, 64, 2>);
-      else launch(logits_kernel<T, HC_SCORE_SNAPKV, 0, 2>);
-    } else {
-      if (D == 128) launch(logits_kernel<T, HC_SCORE_SNAPKV, 128, 4>);
-      else if (D == 64) launch(logits_kernel<T, HC_SCORE_SNAPKV, 64, 4>);
-      else launch(logits_kernel<T, HC_SCORE_SNAPKV, 0, 4>);
+  bool done = false;
+  if constexpr (sizeof(T) == 2) {
+    if (dig) {
+      auto digits = [&](auto kern) {
+        hipLaunchKernelGGL(kern, dim3((unsigned)(lay.wpad / 4), (unsigned)Hk, (unsigned)B), dim3(256), 0, st,
+                           (const T*)q, (const T* const*)q_rows, q_sb, q_sh, q_ss, q_row0, (int)Hq, (int)Hk, (int)W,
+                           (int)lay.wpad, qf, rmax, rstat, qd, qrow);
+      };
+      if (D == 128) digits(qdigit_kernel<T, 128>);
+      else digits(qdigit_kernel<T, 64>);
+      launch_logits_i8<T>(mode, B, Hk, S, D, W, lay.wpad, (const T*)k, (const T* const*)k_rows, k_sb, k_sh,
+                          k_ss, k_bytes, qf, qd, qrow, scal, logits, rmax, st);
+      done = true;
     }
-  } else {
-    // the raw sums' fp64 divides leave no registers for the unrolled ring
-    if (rows == kRowBlk) launch(logits_kernel<T, HC_SCORE_RAWSUM, 0, 2>);
-    else launch(logits_kernel<T, HC_SCORE_RAWSUM, 0, 4>);
+  }
+  if (!done) {
+    hipLaunchKernelGGL(qmean_kernel<T>, dim3((unsigned)lay.wpad, (unsigned)Hk, (unsigned)B),
+                       dim3((unsigned)(D < 64 ? 64 : D)), 0, st, (const T*)q, (const T* const*)q_rows, q_sb, q_sh,
+                       q_ss, q_row0, (int)Hq,
+                       (int)Hk, (int)W, (int)lay.wpad, (int)D, qf, rmax, rstat);
+    const size_t lds = (size_t)(rows * (D + 1) * 8);
+    const int64_t wg1 = cdiv(S, (int64_t)kChunkM) * Hk * nrb * B;  // workgroups at one chunk each
+    const int cpw = (int)std::max<int64_t>(1, std::min<int64_t>(kLogitChunks, wg1 / kLogitTargetWg));
+    const dim3 grid((unsigned)cdiv(S, (int64_t)kChunkM * cpw), (unsigned)(Hk * nrb), (unsigned)B);
+    auto launch = [&](auto kern) {
+      if (lds > 48 * 1024)
+        (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+      hipLaunchKernelGGL(kern, grid, dim3(256), lds, st, (const T*)k, (const T* const*)k_rows, k_sb, k_sh, k_ss,
+                         k_bytes, (const double*)qf,
+                         (int)Hk, (int)S, (int)D, (int)W, (int)lay.wpad, scal, cpw, logits, rmax);
+    };
+    if (mode == HC_SCORE_SNAPKV) {
+      if (rows == kRowBlk) {
+        if (D == 128) launch(logits_kernel<T, HC_SCORE_SNAPKV, 128, 2>);
+        else if (D == 64) launch(logits_kernel<T, HC_SCORE_SNAPKV, 64, 2>);
+        else launch(logits_kernel<T, HC_SCORE_SNAPKV, 0, 2>);
+      } else {
+        if (D == 128) launch(logits_kernel<T, HC_SCORE_SNAPKV, 128, 4>);
+        else if (D == 64) launch(logits_kernel<T, HC_SCORE_SNAPKV, 64, 4>);
+        else launch(logits_kernel<T, HC_SCORE_SNAPKV, 0, 4>);
+      }
+    } else {
+      // the raw sums' fp64 divides leave no registers for the unrolled ring
+      if (rows == kRowBlk) launch(logits_kernel<T, HC_SCORE_RAWSUM, 0, 2>);
+      else launch(logits_kernel<T, HC_SCORE_RAWSUM, 0, 4>);
+    }
   }
   if (mode == HC_SCORE_SNAPKV) {
     // rows split across the waves of a workgroup (1, 2 or 4 per row) when

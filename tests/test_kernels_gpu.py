@@ -583,6 +583,60 @@ def test_snapkv_scores_bit_exact(B, Hq, Hk, S, D, W, dtype, pool, pooling):
     assert torch.equal(got, want), (got - want).abs().max()
 
 
+def _digit_inputs(kind, shape_q, shape_k, dtype):
+    """Queries and keys where the int8 digits of the window logits can go
+    wrong: elements below their window, scales at the types' ends, dot
+    products that cancel, and values that have no digits."""
+    q, k = _randn(shape_q, 81, torch.float32), _randn(shape_k, 82, torch.float32)
+    g = torch.Generator().manual_seed(83)
+    if kind == "outliers":
+        k[..., :3] *= 40.0
+    elif kind == "wide":
+        q, k = (t * torch.exp2(torch.randint(-12, 13, t.shape, generator=g).float()) for t in (q, k))
+    elif kind == "tiny":
+        k *= 1e-6
+        q *= 1e-7
+    elif kind == "huge":
+        k *= 1e4          # below half's largest, 65504, for every |k| < 6.5
+    elif kind == "zeros":
+        k[:, :, ::3] = 0.0
+        q[:, :, -2:] = 0.0
+    elif kind == "ends":          # every magnitude at the last mantissa below a power of two
+        k = torch.sign(k) * (2.0 - 2.0 ** -7)
+    q, k = q.to(dtype), k.to(dtype)
+    if kind == "cancel":          # q.k of halves that cancel exactly
+        h = q.shape[-1] // 2
+        q[..., h:] = q[..., :h]
+        k[..., h:] = -k[..., :h]
+    elif kind == "special":
+        k[:, :, 5, 3] = float("inf")
+        k[:, :, 40, 7] = float("nan")
+        q[:, 0, -1, 2] = float("-inf")
+    return q, k
+
+
+@pytest.mark.parametrize("W,S,D", [(1, 200, 128), (8, 331, 64), (17, 1027, 128), (33, 517, 64), (65, 1100, 128)])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("kind", ["normal", "outliers", "wide", "tiny", "huge", "zeros", "ends", "cancel", "special"])
+def test_window_logits_digits_equal_fp64_chain(kind, dtype, W, S, D):
+    """Groups of three equal query heads have the mean of one of them, bit for
+    bit, and run on the fp64 kernel; groups of one and two run on the digits."""
+    B, Hk = 2, 3
+    q, k = _digit_inputs(kind, (B, Hk, S, D), (B, Hk, S, D), dtype)
+    sc = 1.0 / math.sqrt(D)
+    rep = {G: q.repeat_interleave(G, dim=1).to(DEV) for G in (1, 2, 3)}
+    kd = k.to(DEV)
+    for mode in ("snapkv", "rawsum"):
+        want = ops.snapkv_scores(rep[3], kd, W, sc, 1, "maxpool", mode=mode)
+        for G in (1, 2):
+            got = ops.snapkv_scores(rep[G], kd, W, sc, 1, "maxpool", mode=mode)
+            assert torch.equal(got.view(torch.int32), want.view(torch.int32)) or (
+                kind == "special" and torch.equal(got.isnan(), want.isnan())
+                and torch.equal(got.nan_to_num(), want.nan_to_num())), (mode, G)
+        if kind != "special":
+            assert torch.equal(want.cpu(), ref.window_scores(q, k, W, sc, 1, "maxpool", mode=mode)), mode
+
+
 def test_snapkv_scores_and_keep_llama8b_8k_layer():
     """One layer of the 8k fp16 workload with needles: scores, kept indices
     and the compacted K/V are bit-exact."""
