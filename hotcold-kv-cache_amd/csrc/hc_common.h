@@ -195,6 +195,13 @@ struct DetExp {
     const double p = poly<0>(x, k);
     return x >= -708.0 ? scale(p, k) : 0.0;  // false for -inf and NaN
   }
+  // The contract's value, except that arguments below -708 (-inf and NaN too)
+  // give exp(-708), about 3.3e-308, instead of 0.
+  __device__ __forceinline__ double floored(double x) const {
+    uint32_t k;
+    const double p = poly<0>(x, k);
+    return scale(p, k);
+  }
   // The bits of rint(e * 2^44) + 2^52 for the contract's value e.  e * 2^44 = p * 2^(k+44) exactly, so one add of
   // 2^52 rounds it as fma(e, 2^44, 2^52) would.  Below -708 it uses
   // exp(-708) (~3.3e-308) instead of 0: rint(e * 2^44) is 0 for both.

@@ -89,8 +89,8 @@ struct SumF32 {
 };
 
 // The group-mean queries with their digits: qf[b][h][w][d] as qmean_kernel
-// writes it (zero rows past W), and its resets of the row maxima and the
-// padding statistics.  grid (wpad / 4, Hk, B), block 256, one wave per row;
+// writes it (zero rows past W), and its resets of the row maxima, the NaN flag
+// and the padding statistics.  grid (wpad / 4, Hk, B), block 256, one wave per row;
 // lane l owns dims E l .. E l + E - 1.  A digit byte of row w lies where the B
 // operand reads it: [row block of 16][digit][k-step of 64][lane][16], lane
 // (kk, row) holding dims 8 * (kk + 4 * t) + r of the pieces t = 2s, 2s + 1 of
@@ -102,11 +102,13 @@ __global__ __launch_bounds__(256) void qdigit_kernel(const T* __restrict__ q, co
                                                      int64_t q_sb, int64_t q_sh, int64_t q_ss, int64_t q_row0, int Hq,
                                                      int Hk, int W, int wpad, double* __restrict__ qf,
                                                      uint32_t* __restrict__ rmax, RowStat* __restrict__ rstat,
-                                                     int8_t* __restrict__ qd, QDigitRow* __restrict__ qrow) {
+                                                     uint32_t* __restrict__ nan_flag, int8_t* __restrict__ qd,
+                                                     QDigitRow* __restrict__ qrow) {
   constexpr int E = D / 64;
   const int lane = threadIdx.x & 63, w = (int)blockIdx.x * 4 + (threadIdx.x >> 6), h = blockIdx.y, b = blockIdx.z;
   const int64_t bh = (int64_t)b * Hk + h, row = bh * wpad;
   const int wst = (int)cdiv(W, kStatPad) * kStatPad;
+  if (lane == 0 && w == 0) nan_flag[bh] = 0;
   if (lane == 0 && w < W) rmax[bh * W + w] = order_key(-INFINITY);
   if (lane == 0 && w >= W && w < wst) rstat[bh * wst + w] = RowStat{INFINITY, 0.0};
   double x[E];
@@ -293,7 +295,7 @@ __device__ __forceinline__ void redo_tile(__amdgpu_buffer_rsrc_t krs, uint32_t r
     float L;
     if constexpr (MODE == HC_SCORE_SNAPKV) L = key > qpos0 + w ? -INFINITY : (float)(acc[i] * scaling);
     else L = (float)(acc[i] / scaling);
-    const bool ok = key < S && w < nw;
+    const bool ok = key < ld && w < nw;
     const uint32_t bits = __float_as_uint(L);
     bstore<4>(lrs, ok ? (uint32_t)((w0 + w) * ld + key) * 4u : kOob, &bits);
     m = fmaxf(m, ok ? L : -INFINITY);
@@ -451,7 +453,7 @@ __global__ __launch_bounds__(256, 3) void logits_i8_kernel(
       } else {
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          bstore<4>(lrs, key + i < S ? off + 4u * i : kOob, &bits[i]);   // kOob + 12 is out of range too
+          bstore<4>(lrs, key + i < ld ? off + 4u * i : kOob, &bits[i]);   // kOob + 12 is out of range too
           if constexpr (MODE == HC_SCORE_SNAPKV) mrow[nb] = fmaxf(mrow[nb], ok && key + i < S ? L[i] : -INFINITY);
         }
       }
@@ -484,7 +486,7 @@ __global__ __launch_bounds__(256, 3) void logits_i8_kernel(
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const int w = 16 * nb + col, key = key0 + 4 * kk + i;
-        bstore<4>(lrs, key < S && w < nw ? (uint32_t)((w0 + w) * ld + key) * 4u : kOob, &ninf);
+        bstore<4>(lrs, key < ld && w < nw ? (uint32_t)((w0 + w) * ld + key) * 4u : kOob, &ninf);
       }
     key0 += CHUNK;
   }

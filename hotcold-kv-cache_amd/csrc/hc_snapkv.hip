@@ -32,7 +32,9 @@ constexpr int kNeverRead = 512;  // > the 256 (rowsum) and 270 (imp_pool) read m
 
 // Per window row, for the importance pass: the row max and 1/l_w in fp64.
 // Rows are padded to a multiple of kStatPad per (b, h); the padding rows hold
-// {+inf, 0}, so they add an exact zero to the importance chain.
+// {+inf, 0}, so they add an exact zero to the importance chain.  A row whose
+// sum l_w is 0 (no logit is finite) has inv NaN and raises its head's flag:
+// every score of the head is NaN.
 struct RowStat {
   double m, inv;
 };
@@ -55,20 +57,33 @@ static int64_t row_block(int64_t W) { return W > kRowBlk ? kRowBlkWide : kRowBlk
 constexpr int kMaxPool = 32;  // max half-width of the pooling window
 
 struct ScoreLayout {
-  int64_t wpad, nchunk_m, qf_off, logits_off, rmax_off, rstat_off, qd_off, qrow_off, total;
+  int64_t wpad, nchunk_m, ld, qf_off, logits_off, rmax_off, rstat_off, nan_off, qd_off, qrow_off, total;
 };
 
 static int64_t al256(int64_t x) { return (x + 255) & ~(int64_t)255; }
+
+// Floats per logits row: S rounded up to the 16 keys of a tile, so that rows
+// are 64-byte aligned and the normaliser reads four keys per load at any S (a
+// prompt of 5003: 508 -> 462 us for 32 heads' full-prompt rows); S itself where
+// the padding would take a head's logits past the 2 GiB of a buffer offset.
+// The logits kernels write the padding masked, as keys after every row's
+// position.
+static int64_t logit_ld(int64_t S, int64_t W) {
+  const int64_t ld = cdiv(S, 16) * 16;
+  return W * ld * 4 < ((int64_t)1 << 31) ? ld : S;
+}
 
 static ScoreLayout score_layout(int64_t B, int64_t Hk, int64_t S, int64_t D, int64_t W) {
   ScoreLayout L;
   L.wpad = cdiv(W, row_block(W)) * row_block(W);
   L.nchunk_m = cdiv(S, kChunkM);
+  L.ld = logit_ld(S, W);
   L.qf_off = 0;
   L.logits_off = al256(L.qf_off + B * Hk * L.wpad * D * 8);
-  L.rmax_off = al256(L.logits_off + B * Hk * W * S * 4);
+  L.rmax_off = al256(L.logits_off + B * Hk * W * L.ld * 4);
   L.rstat_off = al256(L.rmax_off + B * Hk * W * 4);
-  L.qd_off = al256(L.rstat_off + B * Hk * cdiv(W, kStatPad) * kStatPad * (int64_t)sizeof(RowStat));
+  L.nan_off = al256(L.rstat_off + B * Hk * cdiv(W, kStatPad) * kStatPad * (int64_t)sizeof(RowStat));
+  L.qd_off = al256(L.nan_off + B * Hk * 4);
   L.qrow_off = al256(L.qd_off + B * Hk * L.wpad * D * kDigits);
   L.total = al256(L.qrow_off + B * Hk * L.wpad * (int64_t)sizeof(QDigitRow));
   return L;
@@ -76,14 +91,17 @@ static ScoreLayout score_layout(int64_t B, int64_t Hk, int64_t S, int64_t D, int
 
 // qf[b][h][w][d] for w < wpad (zero rows past W).  grid (wpad, Hk, B), block D.
 // Also resets the row-max keys (to the key of -inf) that the logits kernel
-// accumulates into, and writes the padding rows of the row statistics.
+// accumulates into and the head's NaN flag (RowStat), and writes the padding
+// rows of the row statistics.
 // q_rows (may be NULL): row b's queries start at q_rows[b] instead of q + b*q_sb.
 template <typename T>
 __global__ void qmean_kernel(const T* __restrict__ q, const T* const* __restrict__ q_rows, int64_t q_sb,
                              int64_t q_sh, int64_t q_ss, int64_t q_row0, int Hq, int Hk, int W, int wpad, int D,
-                             double* __restrict__ qf, uint32_t* __restrict__ rmax, RowStat* __restrict__ rstat) {
+                             double* __restrict__ qf, uint32_t* __restrict__ rmax, RowStat* __restrict__ rstat,
+                             uint32_t* __restrict__ nan_flag) {
   const int w = blockIdx.x, h = blockIdx.y, b = blockIdx.z;
   const int d = threadIdx.x;
+  if (d == 0 && w == 0) nan_flag[(int64_t)b * Hk + h] = 0;
   const int wst = (int)cdiv(W, kStatPad) * kStatPad;  // wst <= wpad
   if (d == 0 && w < W) rmax[((int64_t)b * Hk + h) * W + w] = order_key(-INFINITY);
   if (d == 0 && w >= W && w < wst) rstat[((int64_t)b * Hk + h) * wst + w] = RowStat{INFINITY, 0.0};
@@ -195,7 +213,7 @@ template <typename T, int MODE, int DC, int NRB>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, NRB == 2 ? 4 : 2))) void logits_kernel(
     const T* __restrict__ k, const T* const* __restrict__ k_rows, int64_t k_sb, int64_t k_sh, int64_t k_ss,
     uint32_t k_bytes, const double* __restrict__ qf, int Hk, int S, int Drt, int W, int wpad, double scaling,
-    int cpw, float* __restrict__ logits, uint32_t* __restrict__ rmax) {
+    int cpw, int ldl, float* __restrict__ logits, uint32_t* __restrict__ rmax) {
   constexpr int ROWS = 16 * NRB;  // window rows of the workgroup: NRB 16-row MFMA blocks
   const int D = DC > 0 ? DC : Drt;
   extern __shared__ double sq[];  // [ROWS][D + 1] window-row block of qf
@@ -229,8 +247,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, NRB == 2
   const int qpos0 = S - W + w0;
   const uint32_t sl = KOperand<T>::sel(kk);
   const double* qrow = sq + col * ld + kk;  // row 16 i + col of the block at qrow + 16 i ld
-  // this (b, h)'s W x S logits; W * S * 4 < 2^31 is checked by the host
-  const __amdgpu_buffer_rsrc_t lrs = make_rsrc(logits + bh * W * S, (uint32_t)((int64_t)W * S * 4));
+  // this (b, h)'s W x ldl logits; W * ldl * 4 < 2^31 is checked by the host
+  const __amdgpu_buffer_rsrc_t lrs = make_rsrc(logits + bh * W * ldl, (uint32_t)((int64_t)W * ldl * 4));
   float mrow[4 * NRB];
 #pragma unroll
   for (int j = 0; j < 4 * NRB; ++j) mrow[j] = -INFINITY;
@@ -347,9 +365,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, NRB == 2
           float L;
           if constexpr (MODE == HC_SCORE_SNAPKV) L = (key > qpos0 + w) ? -INFINITY : (float)(v * scaling);
           else L = (float)(v / scaling);
-          const bool ok = key < S && w < nw;
+          const bool ok = key < ldl && w < nw;
           const uint32_t bits = __float_as_uint(L);
-          bstore<4>(lrs, ok ? (uint32_t)((w0 + w) * S + key) * 4u : kOob, &bits);
+          bstore<4>(lrs, ok ? (uint32_t)((w0 + w) * ldl + key) * 4u : kOob, &bits);
           if constexpr (MODE == HC_SCORE_SNAPKV) mrow[4 * nbk + i] = fmaxf(mrow[4 * nbk + i], ok ? L : -INFINITY);
         }
       }
@@ -370,7 +388,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, NRB == 2
         for (int mb = 0; mb < 2; ++mb) {
           const int w = 16 * nbk + kk + 4 * i;
           const int key = key0 + 16 * mb + col;
-          bstore<4>(lrs, (key < S && w < nw) ? (uint32_t)((w0 + w) * S + key) * 4u : kOob, &ninf);
+          bstore<4>(lrs, (key < ldl && w < nw) ? (uint32_t)((w0 + w) * ldl + key) * 4u : kOob, &ninf);
         }
       }
     }
@@ -411,8 +429,9 @@ constexpr int kSumTargetWaves = 2048;
 
 template <bool VEC>
 __global__ __launch_bounds__(256) void rowsum_kernel(const float* __restrict__ logits,
-                                                     const uint32_t* __restrict__ rmax, int Hk, int S, int W,
-                                                     int nsplit, RowStat* __restrict__ rstat) {
+                                                     const uint32_t* __restrict__ rmax, int Hk, int S, int ld, int W,
+                                                     int nsplit, RowStat* __restrict__ rstat,
+                                                     uint32_t* __restrict__ nan_flag) {
   __shared__ uint64_t sm_part[4];
   // the wave index through readfirstlane: the row's buffer resource is then
   // known to be wave-uniform and lives in SGPRs (no waterfall per load)
@@ -424,7 +443,7 @@ __global__ __launch_bounds__(256) void rowsum_kernel(const float* __restrict__ l
   const int64_t bh = (int64_t)blockIdx.z * Hk + blockIdx.y;
   const double md = (double)key_to_float(rmax[bh * W + wr]);
   const DetExp dexp = DetExp::load();
-  const __amdgpu_buffer_rsrc_t rs = make_rsrc(logits + (bh * W + wr) * S, (uint32_t)S * 4u);
+  const __amdgpu_buffer_rsrc_t rs = make_rsrc(logits + (bh * W + wr) * ld, (uint32_t)ld * 4u);
   // this split's steps [st0, st0 + nstep) and keys [st0 * 256, kend); a wave
   // past W streams nothing (kend = 0).  The row attends keys up to its own
   // position S - W + w; later keys are -inf and add only the bias, so the
@@ -433,7 +452,7 @@ __global__ __launch_bounds__(256) void rowsum_kernel(const float* __restrict__ l
   const int sps = (nstep_all + nsplit - 1) / nsplit;
   const int st0 = min(nstep_all, sp * sps);
   const int nstep = live ? min(nstep_all, st0 + sps) - st0 : 0;
-  const int kend = min(S, (st0 + nstep) * 256);
+  const int kend = min(VEC ? ld : S, (st0 + nstep) * 256);
   uint64_t acc[4] = {0, 0, 0, 0};
   uint32_t x[kSumRing][4];
   auto load = [&](uint32_t (&dst)[4], int step) {
@@ -456,7 +475,7 @@ __global__ __launch_bounds__(256) void rowsum_kernel(const float* __restrict__ l
       load(x[(j + kSumRing - 1) % kSumRing], s0 + j + kSumRing - 1);
       const int key = (st0 + s0 + j) * 256 + lane * 4;
       if constexpr (VEC) {
-        // S % 4 == 0 and kend % 4 == 0: the lane's four keys are all in range
+        // ld % 4 == 0 and kend % 4 == 0: the lane's four keys are all in range
         // or all past kend; past it the max becomes +inf, so x = -inf and the
         // term is the bias
         const double mk = key < kend ? md : INFINITY;
@@ -479,8 +498,12 @@ __global__ __launch_bounds__(256) void rowsum_kernel(const float* __restrict__ l
     t += ((uint64_t)rh << 32) | rl;
   }
   RowStat* out = rstat + bh * (cdiv(W, kStatPad) * kStatPad) + w;
+  auto inverse = [&](uint64_t sum) {
+    if (!sum) nan_flag[bh] = 1;
+    return sum ? 1.0 / ((double)sum * 0x1p-44) : (double)NAN;
+  };
   if (nsplit == 1) {  // uniform: no barrier
-    if (live && lane == 0) *out = RowStat{md, 1.0 / ((double)t * 0x1p-44)};
+    if (live && lane == 0) *out = RowStat{md, inverse(t)};
     return;
   }
   if (lane == 0) sm_part[wave] = t;
@@ -488,7 +511,7 @@ __global__ __launch_bounds__(256) void rowsum_kernel(const float* __restrict__ l
   if (live && sp == 0 && lane == 0) {
     uint64_t tot = 0;
     for (int j = 0; j < nsplit; ++j) tot += sm_part[wave + j];
-    *out = RowStat{md, 1.0 / ((double)tot * 0x1p-44)};
+    *out = RowStat{md, inverse(tot)};
   }
 }
 
@@ -499,14 +522,21 @@ __global__ __launch_bounds__(256) void rowsum_kernel(const float* __restrict__ l
 // row's max and 1/l_w are wave-uniform: they come through scalar loads into
 // SGPRs, with no LDS staging and no per-row branch.
 constexpr int kImpRows = 8;
-// Windows from this many rows on take the mirrored-pair importance kernel
-// when there is no pooling (chain lengths then differ by up to W rows).
-constexpr int kMirrorMinW = 1024;
+// Windows from this many rows on take imp_split_kernel when there is no
+// pooling: with the window the prompt it is the faster from the smallest sizes
+// measured (32 heads of 401: 59 -> 18 us, 1001: 128 -> 51).  Observation
+// windows (8 to 64 rows) have keys enough for one thread each.
+constexpr int kSplitMinW = 256;
 
 // One key's importance: the fma chain over rows [wbeg, W) of the logits
 // column at byte offset `base` (kOob for a lane without a key).  Rows are
 // streamed kImpRows at a time with the next group in flight; a group's
-// logits and (scalar) row statistics are issued one group ahead.  Groups
+// logits and (scalar) row statistics are issued one group ahead.  The
+// exponentials are floored at exp(-708) (DetExp::floored, three instructions
+// less than the select to 0): a floored term of 3.3e-308 or less is below half
+// an ulp of any sum that an fp32 result can show, and sums of floored terms
+// alone round to 0 as sums of zeros do.  A row with no positive term (l_w = 0)
+// must give NaN through 0 * inf; its 1/l_w is stored as NaN.  Groups
 // start at multiples of kImpRows and the statistics are padded to kStatPad
 // (a multiple of 2 * kImpRows) rows.
 template <int MODE>
@@ -528,7 +558,7 @@ __device__ __forceinline__ double imp_chain(__amdgpu_buffer_rsrc_t rs, uint32_t 
   };
   double acc = 0.0;
   // rows [w0, w0 + kImpRows); rows past W add an exact zero: their padding
-  // statistics are {+inf, 0}, so x = -inf, e = 0 and fma(0, 0, acc) = acc
+  // statistics are {+inf, 0}, so x = -inf and fma(e, 0, acc) = acc
   // (acc >= +0)
   auto chain = [&](const uint32_t (&x)[kImpRows], const RowStat (&sx)[kImpRows], int w0) {
 #pragma unroll
@@ -536,7 +566,7 @@ __device__ __forceinline__ double imp_chain(__amdgpu_buffer_rsrc_t rs, uint32_t 
       const int w = w0 + r;
       const float L = __uint_as_float(x[r]);
       if constexpr (MODE == HC_SCORE_SNAPKV) {
-        acc = __builtin_fma(dexp((double)L - sx[r].m), sx[r].inv, acc);
+        acc = __builtin_fma(dexp.floored((double)L - sx[r].m), sx[r].inv, acc);
       } else {
         acc = acc + (w < W ? (double)L : 0.0);
       }
@@ -566,8 +596,8 @@ __device__ __forceinline__ int imp_first_row(int kmin, int S, int W) {
 
 template <int MODE>
 __global__ __launch_bounds__(256) void imp_pool_kernel(const float* __restrict__ logits,
-                                                       const RowStat* __restrict__ rstat, int Hk, int S, int W,
-                                                       int P, int pooling, int ksize,
+                                                       const RowStat* __restrict__ rstat, int Hk, int S, int ld,
+                                                       int W, int P, int pooling, int ksize,
                                                        float* __restrict__ scores) {
   const int h = blockIdx.y, b = blockIdx.z;
   const int64_t bh = (int64_t)b * Hk + h;
@@ -576,17 +606,17 @@ __global__ __launch_bounds__(256) void imp_pool_kernel(const float* __restrict__
   __shared__ float sm_imp[256];
   const int s = c0 - P + (int)threadIdx.x;
   const bool sv = s >= 0 && s < S;
-  // W * S * 4 < 2^31 (checked by the host), so every in-range offset is below
+  // W * ld * 4 < 2^31 (checked by the host), so every in-range offset is below
   // 2^31.  A lane outside [0, S) starts at kOob = 2^31: plus a row offset
   // (< 2^31) it stays out of range; rows past W use the row offset kOob, out
   // of range for in-range lanes (and wrapping to offset 0, a harmless read, for
   // the others, whose result is discarded).
-  const __amdgpu_buffer_rsrc_t rs = make_rsrc(logits + bh * W * S, (uint32_t)((int64_t)W * S * 4));
+  const __amdgpu_buffer_rsrc_t rs = make_rsrc(logits + bh * W * ld, (uint32_t)((int64_t)W * ld * 4));
   const uint32_t base = sv ? (uint32_t)s * 4u : kOob;
   const int wst = (int)cdiv(W, kStatPad) * kStatPad;
   const DetExp dexp = DetExp::load();
   const int wbeg = MODE == HC_SCORE_SNAPKV ? imp_first_row(c0 - P, S, W) : 0;
-  const double acc = imp_chain<MODE>(rs, base, (uint32_t)S * 4u, rstat + bh * wst, wst, W, wbeg, dexp);
+  const double acc = imp_chain<MODE>(rs, base, (uint32_t)ld * 4u, rstat + bh * wst, wst, W, wbeg, dexp);
   sm_imp[threadIdx.x] = sv ? (float)acc : 0.f;
   __syncthreads();
   const int t = threadIdx.x;
@@ -611,37 +641,93 @@ __global__ __launch_bounds__(256) void imp_pool_kernel(const float* __restrict__
   scores[bh * S + s] = out;
 }
 
-// Importance without pooling for long windows, keys in mirrored pairs.
-// With a window as long as the prompt (H2O) key s's chain covers the S - s
-// rows at or after its position, so one thread per key leaves the first
-// keys' threads with thousands of rows and the last keys' with a few, and
-// every chain must stay in one thread (its order is part of the scores).
-// Here thread t of workgroup x owns keys a = 256x + t and S - 1 - a: every
-// thread's two chains together cover about S + 1 rows.  The chains and the
-// fp32 result are those of imp_pool_kernel with P = 0, bit for bit.
-// grid (ceil(ceil(S / 2) / 256), Hk, B), block 256.
-__global__ __launch_bounds__(256) void imp_mirror_kernel(const float* __restrict__ logits,
-                                                         const RowStat* __restrict__ rstat, int Hk, int S, int W,
-                                                         float* __restrict__ scores) {
+// Importance without pooling for long windows (H2O: the window is the
+// prompt), one key per lane.  A key's chain runs over up to S rows and must
+// stay in order, so one thread per key leaves the chip with 1.2 waves per SIMD
+// at 32 heads of 5003 keys.  Only the chain's fma is serial, though: here the
+// four waves of a workgroup evaluate the exponentials of kChainRows rows of its
+// 64 keys into LDS, 8 rows each, and one of them (each in turn) runs the chain
+// over those while the others go on to the next rows.  Terms, order and result
+// are those of imp_pool_kernel with P = 0, bit for bit.  Measured at 32 heads
+// of 5003 x 5003 against one thread per mirrored pair of keys: 883 -> 552 us
+// (2001 x 2001: 318 -> 147); what bounds it is fp64 issue.
+// grid (ceil(S / 64), Hk, B), block 256; the keys with the longest chains
+// first.
+constexpr int kChainRows = 32;
+
+__global__ __launch_bounds__(256) void imp_split_kernel(const float* __restrict__ logits,
+                                                        const RowStat* __restrict__ rstat,
+                                                        const uint32_t* __restrict__ nan_flag, int Hk, int S, int ld,
+                                                        int W, float* __restrict__ scores) {
+  static_assert(kChainRows == 4 * kImpRows && kStatPad % kImpRows == 0, "8 rows per wave and step, all or none padded");
+  __shared__ double e[2][kChainRows][64], inv[2][kChainRows];
+  __shared__ double sum[64];
   const int h = blockIdx.y, b = blockIdx.z;
   const int64_t bh = (int64_t)b * Hk + h;
-  const int c0 = blockIdx.x * 256;
-  const int a = c0 + (int)threadIdx.x;
-  const int m = S - 1 - a;                 // the mirrored key
-  const bool av = a <= m, mv = a < m;      // the middle key of an odd S once
-  const __amdgpu_buffer_rsrc_t rs = make_rsrc(logits + bh * W * S, (uint32_t)((int64_t)W * S * 4));
-  const uint32_t rowb = (uint32_t)S * 4u;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int c0 = blockIdx.x * 64, s = c0 + lane;
+  const __amdgpu_buffer_rsrc_t rs = make_rsrc(logits + bh * W * ld, (uint32_t)((int64_t)W * ld * 4));
+  const uint32_t base = s < S ? (uint32_t)s * 4u : kOob, rowb = (uint32_t)ld * 4u;
   const int wst = (int)cdiv(W, kStatPad) * kStatPad;
   const RowStat* st = rstat + bh * wst;
   const DetExp dexp = DetExp::load();
-  const double acc_a = imp_chain<HC_SCORE_SNAPKV>(rs, av ? (uint32_t)a * 4u : kOob, rowb, st, wst, W,
-                                                  imp_first_row(c0, S, W), dexp);
-  // the workgroup's mirrored keys are S - 1 - c0 - 255 .. S - 1 - c0
-  const double acc_m = imp_chain<HC_SCORE_SNAPKV>(rs, mv ? (uint32_t)m * 4u : kOob, rowb, st, wst, W,
-                                                  imp_first_row(max(0, S - 1 - c0 - 255), S, W), dexp);
-  float* out = scores + bh * S;
-  if (av) out[a] = (float)acc_a;
-  if (mv) out[m] = (float)acc_m;
+  // One step's logits and statistics of this wave's rows, in flight a step
+  // ahead.  Rows past W: kOob is out of range for lanes with a key; the others'
+  // reads (wrapping to the head's first rows) are harmless and their sums not
+  // stored.  Rows past wst are not evaluated: their statistics re-read the last.
+  struct Rows {
+    uint32_t l[kImpRows];
+    double m[kImpRows], inv;     // inv: of the row of lane % 8
+  };
+  auto load = [&](Rows& x, int w0) {
+    const int ww = w0 + wave * kImpRows;
+    const RowStat* g = st + min(ww, wst - kImpRows);
+#pragma unroll
+    for (int r = 0; r < kImpRows; ++r)
+      bload<4>(rs, base + (ww + r < W ? (uint32_t)(ww + r) * rowb : kOob), &x.l[r]);
+#pragma unroll
+    for (int r = 0; r < kImpRows; ++r) x.m[r] = g[r].m;
+    x.inv = g[lane % kImpRows].inv;
+  };
+  if (threadIdx.x < 64) sum[lane] = 0.0;
+  int turn = 0;
+  auto step = [&](const Rows& x, int w0) {
+    const int at = wave * kImpRows, buf = turn & 1;
+    if (w0 + at < wst) {           // wave-uniform
+#pragma unroll
+      for (int r = 0; r < kImpRows; ++r) e[buf][at + r][lane] = dexp.floored((double)__uint_as_float(x.l[r]) - x.m[r]);
+      if (lane < kImpRows) inv[buf][at + lane] = x.inv;
+    }
+    __syncthreads();
+    if (wave == (turn & 3)) {
+      double acc = sum[lane];
+      const int n = min(kChainRows, wst - w0);
+      for (int i0 = 0; i0 < n; i0 += kImpRows) {
+        double t[kImpRows], v[kImpRows];
+#pragma unroll
+        for (int r = 0; r < kImpRows; ++r) {
+          t[r] = e[buf][i0 + r][lane];
+          v[r] = inv[buf][i0 + r];
+        }
+#pragma unroll
+        for (int r = 0; r < kImpRows; ++r) acc = __builtin_fma(t[r], v[r], acc);
+      }
+      sum[lane] = acc;
+    }
+    ++turn;
+  };
+  const int wbeg = imp_first_row(c0, S, W);
+  Rows x, y;
+  load(x, wbeg);
+  for (int w0 = wbeg; w0 < W; w0 += 2 * kChainRows) {
+    load(y, w0 + kChainRows);
+    step(x, w0);
+    load(x, w0 + 2 * kChainRows);
+    if (w0 + kChainRows < W) step(y, w0 + kChainRows);     // workgroup-uniform
+  }
+  __syncthreads();
+  // (rows before wbeg add zeros, unless one of them has no finite logit)
+  if (threadIdx.x < 64 && s < S) scores[bh * S + s] = nan_flag[bh] ? NAN : (float)sum[lane];
 }
 
 // out[b][s] = (float)((sum_h (double)x[b][h][s]) / H), h ascending.
@@ -658,7 +744,7 @@ __global__ void head_mean_kernel(const float* __restrict__ x, int H, int S, floa
 constexpr int kDigitTargetWg = 1280;
 
 template <typename T>
-static void launch_logits_i8(int mode, int64_t B, int64_t Hk, int64_t S, int64_t D, int64_t W,
+static void launch_logits_i8(int mode, int64_t B, int64_t Hk, int64_t S, int64_t ld, int64_t D, int64_t W,
                              int64_t wpad, const T* k, const T* const* k_rows, int64_t k_sb, int64_t k_sh,
                              int64_t k_ss, uint32_t k_bytes, const double* qf, const int8_t* qd,
                              const QDigitRow* qrow, double scal, float* logits, uint32_t* rmax, hipStream_t st) {
@@ -668,7 +754,7 @@ static void launch_logits_i8(int mode, int64_t B, int64_t Hk, int64_t S, int64_t
   const dim3 grid((unsigned)cdiv(S, (int64_t)kDigitChunk * cpw), (unsigned)(Hk * nrb), (unsigned)B);
   auto launch = [&](auto kern) {
     hipLaunchKernelGGL(kern, grid, dim3(256), 0, st, k, k_rows, k_sb, k_sh, k_ss, k_bytes, qf, qd, qrow, (int)Hk,
-                       (int)S, (int)W, (int)wpad, scal, cpw, (int)S, logits, rmax);
+                       (int)S, (int)W, (int)wpad, scal, cpw, (int)ld, logits, rmax);
   };
   auto pick = [&](auto dim) {
     constexpr int DC = decltype(dim)::value;
@@ -697,6 +783,7 @@ static void launch_score(const ScoreLayout& lay, char* ws, int mode, int64_t B, 
   RowStat* rstat = reinterpret_cast<RowStat*>(ws + lay.rstat_off);
   const int rows = (int)row_block(W);
   const int nrb = (int)(lay.wpad / rows);
+  uint32_t* nan_flag = reinterpret_cast<uint32_t*>(ws + lay.nan_off);
   int8_t* qd = reinterpret_cast<int8_t*>(ws + lay.qd_off);
   QDigitRow* qrow = reinterpret_cast<QDigitRow*>(ws + lay.qrow_off);
   // The int8 digits serve 2-byte keys of the compiled head dims.  A group
@@ -711,11 +798,11 @@ static void launch_score(const ScoreLayout& lay, char* ws, int mode, int64_t B, 
       auto digits = [&](auto kern) {
         hipLaunchKernelGGL(kern, dim3((unsigned)(lay.wpad / 4), (unsigned)Hk, (unsigned)B), dim3(256), 0, st,
                            (const T*)q, (const T* const*)q_rows, q_sb, q_sh, q_ss, q_row0, (int)Hq, (int)Hk, (int)W,
-                           (int)lay.wpad, qf, rmax, rstat, qd, qrow);
+                           (int)lay.wpad, qf, rmax, rstat, nan_flag, qd, qrow);
       };
       if (D == 128) digits(qdigit_kernel<T, 128>);
       else digits(qdigit_kernel<T, 64>);
-      launch_logits_i8<T>(mode, B, Hk, S, D, W, lay.wpad, (const T*)k, (const T* const*)k_rows, k_sb, k_sh,
+      launch_logits_i8<T>(mode, B, Hk, S, lay.ld, D, W, lay.wpad, (const T*)k, (const T* const*)k_rows, k_sb, k_sh,
                           k_ss, k_bytes, qf, qd, qrow, scal, logits, rmax, st);
       done = true;
     }
@@ -724,7 +811,7 @@ static void launch_score(const ScoreLayout& lay, char* ws, int mode, int64_t B, 
     hipLaunchKernelGGL(qmean_kernel<T>, dim3((unsigned)lay.wpad, (unsigned)Hk, (unsigned)B),
                        dim3((unsigned)(D < 64 ? 64 : D)), 0, st, (const T*)q, (const T* const*)q_rows, q_sb, q_sh,
                        q_ss, q_row0, (int)Hq,
-                       (int)Hk, (int)W, (int)lay.wpad, (int)D, qf, rmax, rstat);
+                       (int)Hk, (int)W, (int)lay.wpad, (int)D, qf, rmax, rstat, nan_flag);
     const size_t lds = (size_t)(rows * (D + 1) * 8);
     const int64_t wg1 = cdiv(S, (int64_t)kChunkM) * Hk * nrb * B;  // workgroups at one chunk each
     const int cpw = (int)std::max<int64_t>(1, std::min<int64_t>(kLogitChunks, wg1 / kLogitTargetWg));
@@ -734,7 +821,7 @@ static void launch_score(const ScoreLayout& lay, char* ws, int mode, int64_t B, 
         (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
       hipLaunchKernelGGL(kern, grid, dim3(256), lds, st, (const T*)k, (const T* const*)k_rows, k_sb, k_sh, k_ss,
                          k_bytes, (const double*)qf,
-                         (int)Hk, (int)S, (int)D, (int)W, (int)lay.wpad, scal, cpw, logits, rmax);
+                         (int)Hk, (int)S, (int)D, (int)W, (int)lay.wpad, scal, cpw, (int)lay.ld, logits, rmax);
     };
     if (mode == HC_SCORE_SNAPKV) {
       if (rows == kRowBlk) {
@@ -759,27 +846,27 @@ static void launch_score(const ScoreLayout& lay, char* ws, int mode, int64_t B, 
     int nsplit = 1;
     while (nsplit < 4 && rows * nsplit * 2 <= kSumTargetWaves && cdiv(S, 256) >= 2 * nsplit) nsplit *= 2;
     const dim3 g((unsigned)cdiv(W, 4 / nsplit), (unsigned)Hk, (unsigned)B);
-    if (S % 4 == 0)
+    if (lay.ld % 4 == 0)
       hipLaunchKernelGGL(rowsum_kernel<true>, g, dim3(256), 0, st, (const float*)logits, (const uint32_t*)rmax,
-                         (int)Hk, (int)S, (int)W, nsplit, rstat);
+                         (int)Hk, (int)S, (int)lay.ld, (int)W, nsplit, rstat, nan_flag);
     else
       hipLaunchKernelGGL(rowsum_kernel<false>, g, dim3(256), 0, st, (const float*)logits, (const uint32_t*)rmax,
-                         (int)Hk, (int)S, (int)W, nsplit, rstat);
+                         (int)Hk, (int)S, (int)lay.ld, (int)W, nsplit, rstat, nan_flag);
   }
-  if (mode == HC_SCORE_SNAPKV && P == 0 && W >= kMirrorMinW) {
-    const dim3 gm((unsigned)cdiv(cdiv(S, 2), 256), (unsigned)Hk, (unsigned)B);
-    hipLaunchKernelGGL(imp_mirror_kernel, gm, dim3(256), 0, st, (const float*)logits, (const RowStat*)rstat,
-                       (int)Hk, (int)S, (int)W, scores);
+  if (mode == HC_SCORE_SNAPKV && P == 0 && W >= kSplitMinW) {
+    hipLaunchKernelGGL(imp_split_kernel, dim3((unsigned)cdiv(S, 64), (unsigned)Hk, (unsigned)B), dim3(256), 0, st,
+                       (const float*)logits, (const RowStat*)rstat, (const uint32_t*)nan_flag, (int)Hk, (int)S,
+                       (int)lay.ld, (int)W, scores);
     return;
   }
   const dim3 gi((unsigned)cdiv(S, 256 - 2 * P), (unsigned)Hk, (unsigned)B);
   if (mode == HC_SCORE_SNAPKV)
     hipLaunchKernelGGL(imp_pool_kernel<HC_SCORE_SNAPKV>, gi, dim3(256), 0, st, (const float*)logits,
-                       (const RowStat*)rstat, (int)Hk, (int)S, (int)W, P, pooling, ksize,
+                       (const RowStat*)rstat, (int)Hk, (int)S, (int)lay.ld, (int)W, P, pooling, ksize,
                        scores);
   else
     hipLaunchKernelGGL(imp_pool_kernel<HC_SCORE_RAWSUM>, gi, dim3(256), 0, st, (const float*)logits,
-                       (const RowStat*)rstat, (int)Hk, (int)S, (int)W, P, pooling, ksize,
+                       (const RowStat*)rstat, (int)Hk, (int)S, (int)lay.ld, (int)W, P, pooling, ksize,
                        scores);
 }
 

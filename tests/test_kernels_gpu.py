@@ -637,6 +637,22 @@ def test_window_logits_digits_equal_fp64_chain(kind, dtype, W, S, D):
             assert torch.equal(want.cpu(), ref.window_scores(q, k, W, sc, 1, "maxpool", mode=mode)), mode
 
 
+@pytest.mark.parametrize("W,S", [(255, 300), (256, 256), (257, 321), (289, 305), (400, 463)])
+@pytest.mark.parametrize("dtype,pool", [(torch.float16, 1), (torch.float32, 1), (torch.bfloat16, 5)])
+def test_long_window_scores_bit_exact(W, S, dtype, pool):
+    """Either side of the window from which the chains are split over waves,
+    with rows short of their padding and a last step of few rows; one query
+    row with no finite logit makes every score NaN, as the oracle's."""
+    q, k = _randn((1, 4, S, 64), 91, dtype), _randn((1, 2, S, 64), 92, dtype)
+    got = ops.snapkv_scores(q.to(DEV), k.to(DEV), W, 0.125, pool, "avgpool").cpu()
+    assert torch.equal(got, ref.window_scores(q, k, W, 0.125, pool, "avgpool"))
+    q[:, 0, S - 3] = float("nan")
+    got = ops.snapkv_scores(q.to(DEV), k.to(DEV), W, 0.125, pool, "avgpool").cpu()
+    want = ref.window_scores(q, k, W, 0.125, pool, "avgpool")
+    assert torch.isnan(got[:, 0]).all() and torch.equal(got.isnan(), want.isnan())
+    assert torch.equal(got.nan_to_num(), want.nan_to_num())
+
+
 def test_snapkv_scores_and_keep_llama8b_8k_layer():
     """One layer of the 8k fp16 workload with needles: scores, kept indices
     and the compacted K/V are bit-exact."""
