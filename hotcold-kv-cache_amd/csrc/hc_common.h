@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 #include <math.h>
+#include <type_traits>
 #include <utility>
 
 #include "hotcold_hip.h"
@@ -292,6 +293,24 @@ __device__ __forceinline__ void bstore(__amdgpu_buffer_rsrc_t r, uint32_t off, c
   }
 }
 
+// Inclusive prefix sum over a wave's lanes by data-parallel moves (row shifts,
+// then row broadcasts): six dependent adds, where six LDS-routed shuffles cost
+// an LDS round trip each.
+__device__ __forceinline__ uint32_t wave_incl_scan(uint32_t x) {
+  auto dpp = [](uint32_t v, auto ctrl, auto rows) {
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, decltype(ctrl)::value, decltype(rows)::value, 0xf, false);
+  };
+  using std::integral_constant;
+  integral_constant<int, 0xf> all;
+  x += dpp(x, integral_constant<int, 0x111>{}, all);                              // row_shr:1
+  x += dpp(x, integral_constant<int, 0x112>{}, all);                              // row_shr:2
+  x += dpp(x, integral_constant<int, 0x114>{}, all);                              // row_shr:4
+  x += dpp(x, integral_constant<int, 0x118>{}, all);                              // row_shr:8
+  x += dpp(x, integral_constant<int, 0x142>{}, integral_constant<int, 0xa>{});    // row_bcast:15
+  x += dpp(x, integral_constant<int, 0x143>{}, integral_constant<int, 0xc>{});    // row_bcast:31
+  return x;
+}
+
 // Wave-aggregated LDS updates.  Radix-select keys mostly share their leading
 // digits, so plain per-lane atomics on one histogram bin or one append counter
 // serialise across the whole workgroup; here each wave issues one atomic for
@@ -300,7 +319,7 @@ __device__ __forceinline__ void hist_add(uint32_t* hist, uint32_t dig, bool acti
   const uint64_t todo = __ballot(active);
   if (!todo) return;
   const int lane = __lane_id(), leader = __ffsll((unsigned long long)todo) - 1;
-  const uint32_t d0 = (uint32_t)__shfl((int)dig, leader);
+  const uint32_t d0 = (uint32_t)__builtin_amdgcn_readlane((int)dig, leader);
   const uint64_t same = __ballot(active && dig == d0);
   if (lane == leader) atomicAdd(&hist[d0], (uint32_t)__popcll(same));
   if (active && dig != d0) atomicAdd(&hist[dig], 1u);
@@ -314,7 +333,7 @@ __device__ __forceinline__ int append_slot(int* counter, bool want) {
   const int lane = __lane_id(), leader = __ffsll((unsigned long long)m) - 1;
   int base = 0;
   if (lane == leader) base = atomicAdd(counter, __popcll(m));
-  base = __shfl(base, leader);
+  base = __builtin_amdgcn_readlane(base, leader);
   return want ? base + __popcll(m & ((1ull << lane) - 1)) : -1;
 }
 

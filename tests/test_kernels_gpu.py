@@ -695,6 +695,19 @@ def test_rawsum_scores_and_head_mean():
     assert torch.equal(ops.head_mean(got).cpu(), ref.head_mean(want))
 
 
+@pytest.mark.parametrize("S", [33, 64 + 31, 96, 1024 + 31, 1056, 8192 + 33, 32768 + 32, 32768 + 33])
+@pytest.mark.parametrize("levels", [1, 3, 1 << 20])
+def test_keep_index_walk_edges(S, levels):
+    """Prefixes around whole 64-key walks, whole passes of the workgroup and
+    the keys it caches; one value (ties alone decide), three, or all distinct."""
+    g = torch.Generator().manual_seed(S)
+    sc = torch.randint(0, levels, (1, 2, S), generator=g).float() / 3.0
+    for budget in (33, 40, S - 1, S):
+        got, gev = ops.keep_index(sc.to(DEV), 32, budget, return_evicted=True)
+        want, wev = ref.keep_index(sc, 32, budget, return_evicted=True)
+        assert torch.equal(got.cpu(), want) and torch.equal(gev.cpu(), wev), budget
+
+
 @pytest.mark.parametrize("S,window,budget", [(200, 16, 64), (100, 8, 30), (50, 32, 20), (10, 32, 512),
                                              (8192, 32, 512), (5000, 64, 5000), (4097, 1, 2)])
 def test_keep_index_matches_oracle(S, window, budget):
@@ -1425,6 +1438,36 @@ def test_device_index_fp16_pass_equals_the_exact_scan(R):
         dix.search(qd, R, h16)
         dix.search(qd, R, h64, pass16=False)
         assert torch.equal(h16, h64), i
+
+
+@pytest.mark.parametrize("D,tokens,R", [(32, 1, 4), (64, 63, 64), (128, 1024, 1), (96, 1025, 100), (128, 16384, 64),
+                                        (128, 16385, 1024), (64, 40000, 256), (160, 3000, 33)])
+def test_device_index_fp16_pass_sizes(D, tokens, R):
+    """The selection after the fp16 pass at the edges of what it holds in
+    registers, of its lanes per candidate and of its ranks, against the exact
+    scan; then with 5000 vectors whose scores lie within three bins of its
+    histogram, more than it re-scores from a bin alone."""
+    from hotcold_kv.device_index import DeviceIndex
+    g = torch.Generator().manual_seed(tokens)
+    kpre = torch.randn((1, 2, tokens, D), generator=g)
+    q = torch.randn((1, 2, D), generator=g)
+    if tokens > 5000:
+        u = q / q.norm(dim=-1, keepdim=True)
+        w = torch.randn((1, 2, 5000, D), generator=g)
+        w = w - (w * u[:, :, None]).sum(-1, keepdim=True) * u[:, :, None]
+        w = w / w.norm(dim=-1, keepdim=True)
+        c = 0.9 + 0.003 * torch.rand((1, 2, 5000, 1), generator=g)
+        near = kpre.clone()
+        near[:, :, 100:5100] = c * u[:, :, None] + (1 - c * c).sqrt() * w
+    hits = [torch.empty((1, 2, R), dtype=torch.int64, device=DEV) for _ in range(2)]
+    for k in [kpre] + ([near] if tokens > 5000 else []):
+        dix = DeviceIndex(1, 2, D, D, 2, tokens, DEV)
+        dix.add(k.to(DEV), np.arange(tokens, dtype=np.int64)[None])
+        dix.search(q.to(DEV), R, hits[0])
+        dix.search(q.to(DEV), R, hits[1], pass16=False)
+        assert torch.equal(hits[0], hits[1])
+        assert (hits[0][..., min(R, tokens):] == -1).all() and (hits[0][..., :min(R, tokens)] >= 0).all()
+
 
 @pytest.mark.parametrize("per_head,faiss_dim,normalize", [(False, 32, True), (True, 64, True), (True, 96, True),
                                                          (True, 64, False)])
