@@ -749,6 +749,8 @@ def snapkv_scores(q_post, keys, window_size, scaling, kernel_size=7, pooling="ma
 def row_addresses(tensors):
     """Base address of every batch row of every tensor, in order (tensor 0
     rows 0..B-1, tensor 1 rows 0..B-1, ...)."""
+    if all(t.shape[0] == 1 for t in tensors):
+        return [t.data_ptr() for t in tensors]
     ptrs = []
     for t in tensors:
         base, step = t.data_ptr(), t.stride(0) * t.element_size()
@@ -792,19 +794,31 @@ def snapkv_scores_rows(q_list, k_list, window_size, scaling, kernel_size=7, pool
     _same_layout(q_list, "snapkv_scores_rows (queries)")
     _same_layout(k_list, "snapkv_scores_rows (keys)")
     q0, k0 = q_list[0], k_list[0]
+    W = check_score_rows(q0, k0, window_size)
+    if tables is None:
+        tables = device_tables(row_addresses(q_list), row_addresses(k_list), device=k0.device)
+    return score_rows(q0, k0, len(k_list) * q0.shape[0], W, scaling, kernel_size, pooling, *tables)
+
+
+def check_score_rows(q0, k0, window_size):
+    """What snapkv_scores_rows asks of each (queries, keys) pair; the window."""
+    _require_device(q0, k0)
     if q0.dim() != 4 or k0.dim() != 4 or q0.stride(-1) != 1 or k0.stride(-1) != 1:
         raise RuntimeError("snapkv_scores_rows: 4D tensors with contiguous rows required")
     if k0.dtype != q0.dtype:
         raise RuntimeError("snapkv_scores_rows: q and keys must share a dtype")
-    B, Hq, T, D = q0.shape
+    W = min(int(window_size), k0.shape[2])
+    if q0.shape[2] < W:
+        raise RuntimeError(f"snapkv_scores_rows: {q0.shape[2]} query rows hold less than the window {W}")
+    return W
+
+
+def score_rows(q0, k0, R, W, scaling, kernel_size, pooling, qt, kt):
+    """snapkv_scores_rows' launch: R batch rows at the device addresses of the
+    tables qt and kt, laid out as q0 and k0 are (checked by the caller)."""
+    _, Hq, T, D = q0.shape
     _, Hk, S, _ = k0.shape
-    W = min(int(window_size), S)
-    if T < W:
-        raise RuntimeError(f"snapkv_scores_rows: {T} query rows hold less than the window {W}")
-    R = len(k_list) * B
     pool = N.HC_POOL_AVG if pooling == "avgpool" else N.HC_POOL_MAX
-    qt, kt = tables if tables is not None else device_tables(row_addresses(q_list), row_addresses(k_list),
-                                                             device=k0.device)
     scores = torch.empty((R, Hk, S), dtype=torch.float32, device=k0.device)
     lib = N.lib()
     ws = _workspace("score", k0.device, lib.hc_snapkv_score_workspace_size(R, Hk, S, D, W))
@@ -834,21 +848,35 @@ def gather_rows_tab(idx, k_src, v_src, k_dst, v_dst, dst_row0=0, tables=None):
     R = len(k_src) * B
     if idx.dim() != 3 or idx.shape[0] != R or idx.shape[1] != H or idx.stride(-1) != 1:
         raise RuntimeError(f"gather_rows_tab: index {tuple(idx.shape)} must be ({R},{H},n) with unit last stride")
-    n = idx.shape[2]
-    for s, d in ((k_src[0], k_dst[0]), (v_src[0], v_dst[0])):
+    check_gather_rows(s0, v_src[0], d0, v_dst[0], dst_row0 + idx.shape[2])
+    tabs = tables if tables is not None else device_tables(*[row_addresses(x) for x in lists], device=s0.device)
+    gather_rows_at(idx, s0, v_src[0], d0, v_dst[0], tabs, dst_row0)
+
+
+def check_gather_rows(s0, vs, d0, vd, rows):
+    """What gather_rows_tab asks of each set of sources and destinations, the
+    destinations holding at least `rows` rows."""
+    _require_device(s0, vs, d0, vd)
+    B, H, _, D = s0.shape
+    for s, d in ((s0, d0), (vs, vd)):
         if s.dtype != s0.dtype or d.dtype != s0.dtype or s.shape[:2] != (B, H) or d.shape[:2] != (B, H) \
                 or s.shape[3] != D or d.shape[3] != D or s.stride(-1) != 1 or d.stride(-1) != 1:
             raise RuntimeError("gather_rows_tab: K/V sources and destinations do not match")
-        if d.shape[2] < dst_row0 + n:
-            raise RuntimeError(f"gather_rows_tab: destination holds {d.shape[2]} rows, needs {dst_row0 + n}")
-    dev = s0.device
-    tabs = tables if tables is not None else device_tables(*[row_addresses(x) for x in lists], device=dev)
-    vs, vd = v_src[0], v_dst[0]
+        if d.shape[2] < rows:
+            raise RuntimeError(f"gather_rows_tab: destination holds {d.shape[2]} rows, needs {rows}")
+
+
+def gather_rows_at(idx, s0, vs, d0, vd, tabs, dst_row0=0):
+    """gather_rows_tab's launch: the rows at the device addresses of the
+    tables, laid out as k source s0, v source vs, k destination d0 and v
+    destination vd are (checked by the caller)."""
+    R, H, n = idx.shape
+    S, D = s0.shape[2:]
     rc = N.lib().hc_gather_rows_tab(
         R, H, n, D, s0.element_size(), _ptr(idx), idx.stride(0), idx.stride(1), S, int(dst_row0),
         _ptr(tabs[0]), s0.stride(1), s0.stride(2), _ptr(tabs[2]), d0.stride(1), d0.stride(2),
         _ptr(tabs[1]), vs.stride(1), vs.stride(2), _ptr(tabs[3]), vd.stride(1), vd.stride(2),
-        _stream_handle(dev))
+        _stream_handle(s0.device))
     N.check(rc, "hc_gather_rows_tab")
 
 
