@@ -7,7 +7,9 @@
 // weight into seven int32 accumulators (at most 4 * 128 * 2^14 = 2^23 each),
 // so the 62-bit integer dot product is exact.  It differs from the defining
 // fp64 fma chain only by
-//   * the chain's own roundings: at most about D * 2^-53 * ||q|| * ||k||;
+//   * the chain's own roundings: 2^-53 of every partial sum, which together are
+//     at most 2^-53 * ||q'|| * ||k|| with q'_d = (D - d) q_d (a product is in
+//     D - d partial sums), about 0.58 D * ||q|| for even elements;
 //   * query digits below the window: at most (sum of the residuals) * ||k||;
 //   * key digits below the window: such a tile's bound is taken as infinite.
 // With delta the sum of these, a logit whose dot product -delta and +delta
@@ -18,14 +20,16 @@
 // What it buys: the fp64 matrix rate is 32 flop per cycle and SIMD, 1/64 of
 // int8's, so 16 products cost a quarter of the one fp64 product.  Kernel times
 // (fp64 form -> this one, 8 KV heads of 128): window 64, 32k keys x 16 rows
-// f16 1243 -> 713 us, 64k x 4 bf16 with outlier channels 650 -> 470; window
-// 32, 32 layers of 8k keys 343 -> 221, one layer 21.6 -> 19.9 (bound by
-// latency); 32 heads of 5003 x 5003 (H2O) 1977 -> 1217.  What bounds it is
-// vector issue: per 16 keys x 64 rows about 270 instructions make the key
+// f16 1243 -> 685 us, 64k x 4 bf16 with outlier channels 650 -> 419; window
+// 32, 32 layers of 8k keys 343 -> 207, one layer 21.6 -> 19.9 (bound by
+// latency); 32 heads of 5003 x 5003 (H2O) 1977 -> 1172.  What bounds it:
+// vector issue (per 16 keys x 64 rows about 270 instructions make the key
 // digits and 350 the logits, beside 128 matrix instructions of 16 cycles that
-// hide two vector instructions each.  Measured no faster: two key tiles per
-// wave, four waves per SIMD (spills), and a row block's products interleaved
-// with the logits of the one before.
+// hide two vector instructions each) and the logits' stores, which are 14% of
+// the 32k launch and 27% of the H2O one.  Measured no faster: two key tiles
+// per wave, four waves per SIMD (spills), a row block's products interleaved
+// with the logits of the one before, and the keys' digits made once for all
+// row blocks.
 #pragma once
 #include <type_traits>
 
@@ -42,11 +46,14 @@ constexpr uint32_t kBalance = 0x80808080u;   // digits of u: the bytes of (u + k
 constexpr uint32_t kFixMax = 0x7f7f7f7fu;    // the largest value that four balanced digits hold
 
 // Per window row, beside its digits: the scale 2^-sh of its fixed point, and
-// upper bounds of the row's 2-norm and of the sum of its residuals.
+// upper bounds of 2^53 times the roundings' share of delta against a key of
+// 2-norm 1 (||q'|| and kEvalUlps ||q|| for the evaluation's own) and of the sum
+// of its residuals.
 struct QDigitRow {
   double scale;
   float norm, resid;
 };
+constexpr int kEvalUlps = 16;
 
 // Reductions over a wave's lanes: rows (col, col + 16, col + 32, col + 48) by
 // gfx950's row swaps, the 16 lanes of a row by rotations.
@@ -132,7 +139,8 @@ __global__ __launch_bounds__(256) void qdigit_kernel(const T* __restrict__ q, co
   for (int e = 0; e < E; ++e) {
     qf[(row + w) * D + lane * E + e] = x[e];
     hi = max(hi, (uint32_t)__double2hiint(x[e]) & 0x7fffffffu);
-    ss = fmaf((float)x[e], (float)x[e], ss);
+    const float xw = (float)x[e] * (float)(D - (lane * E + e) + kEvalUlps);
+    ss = fmaf(xw, xw, ss);
   }
   hi = reduce_cols(reduce_rows(hi, MaxU32{}), MaxU32{});
   // |x| < 2^(ex + 1), and below kFixMax / 2^30 * 2^ex if the top mantissa bits allow
@@ -276,18 +284,19 @@ __device__ __forceinline__ void redo_tile(__amdgpu_buffer_rsrc_t krs, uint32_t r
   const double* qr = qf + col * D + kk;   // zero rows past the window
   const int w = wt + col;
   doublex4 acc = {0.0, 0.0, 0.0, 0.0};
-  for (int t0 = 0; t0 < D / 4; t0 += 8) {
-    uint32_t kw[8];
-    double q[8];
+  // every operand in flight at once: in four batches the loads' round trips
+  // were most of the tile's time (with the tighter norm of QDigitRow 4% of the
+  // f16 launches' time and 10% of the bf16 one's)
+  uint32_t kw[D / 4];
+  double q[D / 4];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      kw[j] = __builtin_amdgcn_raw_buffer_load_b16(krs, (int)koff, (t0 + j) * 8, 0);
-      q[j] = qr[(t0 + j) * 4];
-    }
-#pragma unroll
-    for (int j = 0; j < 8; ++j)
-      acc = __builtin_amdgcn_mfma_f64_16x16x4f64((double)KFix<T>::get(kw[j], 0), q[j], acc, 0, 0, 0);
+  for (int t = 0; t < D / 4; ++t) {
+    kw[t] = __builtin_amdgcn_raw_buffer_load_b16(krs, (int)koff, t * 8, 0);
+    q[t] = qr[t * 4];
   }
+#pragma unroll
+  for (int t = 0; t < D / 4; ++t)
+    acc = __builtin_amdgcn_mfma_f64_16x16x4f64((double)KFix<T>::get(kw[t], 0), q[t], acc, 0, 0, 0);
   float m = -INFINITY;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {   // keys kk + 4i, row col
@@ -360,8 +369,7 @@ __global__ __launch_bounds__(256, 3) void logits_i8_kernel(
     if (tid < ROWS) {
       const QDigitRow r = qrow[bh * wpad + w0 + tid];
       ssc[tid] = r.scale * lscale;
-      // chain and evaluation roundings, D + 16 of 2^-53 each, and the residuals
-      double dl = (double)r.norm * ((D + 16) * 0x1p-53) + (double)r.resid;
+      double dl = (double)r.norm * 0x1p-53 + (double)r.resid;
 #pragma unroll
       for (int o = 8; o > 0; o >>= 1) dl = fmax(dl, __shfl_xor(dl, o, 64));
       if (col == 0) sdel[tid >> 4] = dl * fabs(lscale) * 1.001;
