@@ -44,6 +44,11 @@ __device__ __forceinline__ int block_excl_scan(int v, int* sm_wave, int* total) 
   return before + incl - v;
 }
 
+// base plus the number of lanes below this one in m.
+__device__ __forceinline__ int lanes_below(uint64_t m, int base) {
+  return (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, (uint32_t)base));
+}
+
 // Digit search of one radix pass over kDigitBins bins: the largest digit d
 // with count(digits > d) < krem <= count(digits >= d).  Thread t holds the
 // bin pair kDigitBins-1-2t, kDigitBins-2-2t, so thread order is descending
@@ -170,7 +175,6 @@ __global__ __launch_bounds__(kTopkThreads) void topk_keep_kernel(const float* __
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int run = (prefix + kTopkThreads - 1) / kTopkThreads * 64;
   const int i0 = min(prefix, wave * run), i1 = min(prefix, i0 + run);
-  const uint64_t below = (1ull << lane) - 1;
   auto walk = [&](auto&& f) {     // f(first key of the 64, their order keys, lane in range)
     for (int c = i0; c < i1; c += 64 * kTopkU) {
       uint32_t ks[kTopkU] = {};
@@ -199,14 +203,16 @@ __global__ __launch_bounds__(kTopkThreads) void topk_keep_kernel(const float* __
   }
   int pos = gt_seen + min(eq_seen, need_eq);
   walk([&](int c, uint32_t k, bool in) {
-    const bool eq = in && k == tkey && keep_prefix > 0;
-    const uint64_t me = __ballot(eq);
-    const bool sel = keep_prefix > 0 && in && (k > tkey || (eq && eq_seen + __popcll(me & below) < need_eq));
+    bool sel = keep_prefix > 0 && in && k > tkey;
+    const uint64_t me = keep_prefix > 0 ? __ballot(in && k == tkey) : 0;
+    if (me) {       // wave-uniform; most 64 keys hold no tie
+      sel = sel || ((me >> lane & 1) && lanes_below(me, eq_seen) < need_eq);
+      eq_seen += __popcll(me);
+    }
     const uint64_t ms = __ballot(sel);
-    const int i = c + lane, at = pos + __popcll(ms & below);   // at: kept indices below i
+    const int i = c + lane, at = lanes_below(ms, pos);   // at: kept indices below i
     if (sel) out[at] = i;
     else if (ev && in) ev[i - at] = i;
-    eq_seen += __popcll(me);
     pos += __popcll(ms);
   });
   for (int j = threadIdx.x; j < window; j += kTopkThreads) out[keep_prefix + j] = prefix + j;
