@@ -87,7 +87,7 @@ __device__ __forceinline__ void find_digit(const uint32_t* hist, uint32_t krem, 
 // moves, the histograms' leaders on lane reads, and the kept indices come from
 // ballots over 64 consecutive keys (each through an LDS shuffle, and runs of
 // keys per thread, took 17.3 us for 8 rows of 8160 keys and 26.8 for one of
-// 16352; this 15.0 and 20.7).
+// 16352; this 14.8 and 20.3).
 __global__ __launch_bounds__(kTopkThreads) void topk_keep_kernel(const float* __restrict__ scores, int64_t s_sb,
                                                                  int64_t s_sh, int H, int prefix, int keep_prefix,
                                                                  int window, int64_t* __restrict__ keep,
