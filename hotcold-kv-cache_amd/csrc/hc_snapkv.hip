@@ -596,7 +596,8 @@ __device__ __forceinline__ int imp_first_row(int kmin, int S, int W) {
 
 template <int MODE>
 __global__ __launch_bounds__(256) void imp_pool_kernel(const float* __restrict__ logits,
-                                                       const RowStat* __restrict__ rstat, int Hk, int S, int ld,
+                                                       const RowStat* __restrict__ rstat,
+                                                       const uint32_t* __restrict__ nan_flag, int Hk, int S, int ld,
                                                        int W, int P, int pooling, int ksize,
                                                        float* __restrict__ scores) {
   const int h = blockIdx.y, b = blockIdx.z;
@@ -617,7 +618,10 @@ __global__ __launch_bounds__(256) void imp_pool_kernel(const float* __restrict__
   const DetExp dexp = DetExp::load();
   const int wbeg = MODE == HC_SCORE_SNAPKV ? imp_first_row(c0 - P, S, W) : 0;
   const double acc = imp_chain<MODE>(rs, base, (uint32_t)ld * 4u, rstat + bh * wst, wst, W, wbeg, dexp);
-  sm_imp[threadIdx.x] = sv ? (float)acc : 0.f;
+  float imp = (float)acc;
+  // (rows before wbeg add zeros, unless one of them has no finite logit)
+  if constexpr (MODE == HC_SCORE_SNAPKV) imp = nan_flag[bh] ? NAN : imp;
+  sm_imp[threadIdx.x] = sv ? imp : 0.f;
   __syncthreads();
   const int t = threadIdx.x;
   if (t < P || t >= 256 - P || s >= S) return;
@@ -862,12 +866,12 @@ static void launch_score(const ScoreLayout& lay, char* ws, int mode, int64_t B, 
   const dim3 gi((unsigned)cdiv(S, 256 - 2 * P), (unsigned)Hk, (unsigned)B);
   if (mode == HC_SCORE_SNAPKV)
     hipLaunchKernelGGL(imp_pool_kernel<HC_SCORE_SNAPKV>, gi, dim3(256), 0, st, (const float*)logits,
-                       (const RowStat*)rstat, (int)Hk, (int)S, (int)lay.ld, (int)W, P, pooling, ksize,
-                       scores);
+                       (const RowStat*)rstat, (const uint32_t*)nan_flag, (int)Hk, (int)S, (int)lay.ld, (int)W, P,
+                       pooling, ksize, scores);
   else
     hipLaunchKernelGGL(imp_pool_kernel<HC_SCORE_RAWSUM>, gi, dim3(256), 0, st, (const float*)logits,
-                       (const RowStat*)rstat, (int)Hk, (int)S, (int)lay.ld, (int)W, P, pooling, ksize,
-                       scores);
+                       (const RowStat*)rstat, (const uint32_t*)nan_flag, (int)Hk, (int)S, (int)lay.ld, (int)W, P,
+                       pooling, ksize, scores);
 }
 
 }  // namespace hc

@@ -653,6 +653,20 @@ def test_long_window_scores_bit_exact(W, S, dtype, pool):
     assert torch.equal(got.nan_to_num(), want.nan_to_num())
 
 
+@pytest.mark.parametrize("W,S,pool,pooling", [(64, 8270, 7, "avgpool"), (64, 8270, 7, "maxpool"), (64, 8232, 1, "maxpool"),
+                                              (256, 8400, 5, "avgpool")])
+def test_early_row_without_finite_logit_makes_every_score_nan(W, S, pool, pooling):
+    """The workgroup of the last keys starts its chains past an early window
+    row; a row with no finite logit is still 0 * inf in every key's chain."""
+    q, k = _randn((1, 2, S, 64), 93, torch.float16), _randn((1, 2, S, 64), 94, torch.float16)
+    q[:, 0, S - W + 5] = float("nan")
+    got = ops.snapkv_scores(q.to(DEV), k.to(DEV), W, 0.125, pool, pooling).cpu()
+    want = ref.window_scores(q, k, W, 0.125, pool, pooling)
+    assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.nan_to_num(), want.nan_to_num())
+    if pooling == "avgpool":
+        assert torch.isnan(got[:, 0]).all() and not torch.isnan(got[:, 1]).any()
+
+
 def test_snapkv_scores_and_keep_llama8b_8k_layer():
     """One layer of the 8k fp16 workload with needles: scores, kept indices
     and the compacted K/V are bit-exact."""
