@@ -10,20 +10,24 @@
 //   * the chain's own roundings: 2^-53 of every partial sum, which together are
 //     at most 2^-53 * ||q'|| * ||k|| with q'_d = (D - d) q_d (a product is in
 //     D - d partial sums), about 0.58 D * ||q|| for even elements;
-//   * query digits below the window: at most (sum of the residuals) * ||k||;
-//   * key digits below the window: such a tile's bound is taken as infinite.
+//   * query digits below the window: at most (sum of the residuals) * ||k||.
 // With delta the sum of these, a logit whose dot product -delta and +delta
 // round to one float is that float; a 16 x 16 tile with any other logit is
-// recomputed by the fp64 chain itself (redo_tile).  Infinities and NaN take
-// the same way.  On N(0,1) prompts about 1% of the tiles are redone (22.9k of
-// 1.6M in the H2O launch below, before the bound was weighted by q').
+// recomputed by the fp64 chain itself (chain_tiles): 0.7 to 0.8% of the tiles of
+// N(0,1) prompts, a count over 12000.
+//
+// Keys with bits below the window (f16 tiles of wide channels, a bf16 tile in
+// some hundred) take a fifth digit, four more products (KDigits::low).  What
+// has no digits goes to the chain without them: tiles beyond five digits,
+// infinities and NaN, and every tile of a workgroup whose query rows have
+// residuals that would leave most of its tiles open (kOpenRatio).
 //
 // What it buys: the fp64 matrix rate is 32 flop per cycle and SIMD, 1/64 of
 // int8's, so 16 products cost a quarter of the one fp64 product.  Kernel times
 // (fp64 form -> this one, 8 KV heads of 128): window 64, 32k keys x 16 rows
-// f16 1243 -> 685 us, 64k x 4 bf16 with outlier channels 650 -> 419; window
-// 32, 32 layers of 8k keys 343 -> 207, one layer 21.6 -> 19.9 (bound by
-// latency); 32 heads of 5003 x 5003 (H2O) 1977 -> 1172.  What bounds it:
+// f16 1243 -> 685 us, 64k x 4 bf16 with outlier channels 650 -> 400; window
+// 32, 32 layers of 8k keys 343 -> 207, one layer 21.6 -> 19.5 (bound by
+// latency); 32 heads of 5003 x 5003 (H2O) 1977 -> 1100.  What bounds it:
 // vector issue (per 16 keys x 64 rows about 270 instructions make the key
 // digits and 350 the logits, beside 128 matrix instructions of 16 cycles that
 // hide two vector instructions each) and the logits' stores, which are 14% of
@@ -31,6 +35,14 @@
 // per wave, four waves per SIMD (spills), a row block's products interleaved
 // with the logits of the one before, and the keys' digits made once for all
 // row blocks.
+//
+// Off the common path (f16, 8 KV heads, the whole score call, against the fp64
+// form; 32k keys x 4 rows, window 64 | 8k x 32, window 32): four channels 100
+// times wider 411 -> 338 us | -, 400 times 412 -> 377 | 459 -> 447; a query
+// channel 100 times wider 409 -> 407 | 450 -> 390, 1000 times 409 -> 457 | 451 ->
+// 426; exponents over 24 binades 415 -> 460 | 453 -> 430.  So where all tiles are
+// the chain's it is from 6% faster to 12% slower than the fp64 kernel, whose
+// loop it is without that kernel's LDS for the whole window.
 #pragma once
 #include <type_traits>
 
@@ -39,6 +51,7 @@
 namespace hc {
 
 typedef int i32x4 __attribute__((ext_vector_type(4)));
+typedef double doublex2 __attribute__((ext_vector_type(2)));
 typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
 
 constexpr int kDigitChunk = 64;              // keys per workgroup and step: 4 waves x 16
@@ -55,6 +68,14 @@ struct QDigitRow {
   float norm, resid;
 };
 constexpr int kEvalUlps = 16;
+// A row whose residuals are r of its norm leaves about 2^34 r of its logits
+// open (delta over half an ulp of a logit of typical size, head dim 128).  From
+// this sum of r over a row block on, the mean over a workgroup's, all its tiles
+// go to the chain.  Measured with one query channel 60 to 1000 times wider (f16,
+// 8k keys x 32 rows, window 32): 371, 390, 432, 435, 426 us where a bound of
+// 2^-39 gives 413, 441, 505, 488, 458; at 32k x 4, window 64, the two differ by
+// at most 6% either way.
+constexpr float kOpenRatio = 0x1p-41f;
 
 // Reductions over a wave's lanes: rows (col, col + 16, col + 32, col + 48) by
 // gfx950's row swaps, the 16 lanes of a row by rotations.
@@ -96,15 +117,17 @@ struct SumF32 {
   }
 };
 
-// The group-mean queries with their digits: qf[b][h][w][d] as qmean_kernel
-// writes it (zero rows past W), and its resets of the row maxima, the NaN flag
-// and the padding statistics.  grid (wpad / 4, Hk, B), block 256, one wave per row;
-// lane l owns dims E l .. E l + E - 1.  A digit byte of row w lies where the B
-// operand reads it: [row block of 16][digit][k-step of 64][lane][16], lane
-// (kk, row) holding dims 8 * (kk + 4 * t) + r of the pieces t = 2s, 2s + 1 of
-// k-step s.  Bound by its stores (the fp64 means and 4 bytes of digits per
-// element): 99 us for 32 heads of 5003 rows, 78 without the digits; a block of
-// D threads per row with bounds reduced in fp64 across waves took 170.
+// The group-mean queries with their digits, and qmean_kernel's resets of the
+// row maxima, the NaN flag and the padding statistics (zero rows past W).
+// grid (wpad / 4, Hk, B), block 256, one wave per row; lane l owns dims
+// E l .. E l + E - 1.  Both leave in the order that the matrix instructions read
+// them, 16 rows to a block, through LDS so that four rows' 16-byte pieces go out
+// together:
+//   qf [row block][dims 8u .. 8u + 7][lane][2], lane (kk, row) holding dims
+//      8u + kk and 8u + 4 + kk: two k-steps of the fp64 chain;
+//   qd [row block][digit][k-step of 64][lane][16], lane (kk, row) holding dims
+//      8 * (kk + 4 * t) + r of the pieces t = 2s, 2s + 1 of k-step s.
+// Bound by its stores (12 bytes per element).
 template <typename T, int D>
 __global__ __launch_bounds__(256) void qdigit_kernel(const T* __restrict__ q, const T* const* __restrict__ q_rows,
                                                      int64_t q_sb, int64_t q_sh, int64_t q_ss, int64_t q_row0, int Hq,
@@ -113,7 +136,10 @@ __global__ __launch_bounds__(256) void qdigit_kernel(const T* __restrict__ q, co
                                                      uint32_t* __restrict__ nan_flag, int8_t* __restrict__ qd,
                                                      QDigitRow* __restrict__ qrow) {
   constexpr int E = D / 64;
-  const int lane = threadIdx.x & 63, w = (int)blockIdx.x * 4 + (threadIdx.x >> 6), h = blockIdx.y, b = blockIdx.z;
+  __shared__ double sx[4][D + 4];
+  __shared__ i32x4 sd[D * kDigits / 4];
+  const int tid = threadIdx.x, lane = tid & 63, r = tid >> 6;
+  const int w = (int)blockIdx.x * 4 + r, h = blockIdx.y, b = blockIdx.z;
   const int64_t bh = (int64_t)b * Hk + h, row = bh * wpad;
   const int wst = (int)cdiv(W, kStatPad) * kStatPad;
   if (lane == 0 && w == 0) nan_flag[bh] = 0;
@@ -138,7 +164,7 @@ __global__ __launch_bounds__(256) void qdigit_kernel(const T* __restrict__ q, co
   float ss = 0.f;
 #pragma unroll
   for (int e = 0; e < E; ++e) {
-    qf[(row + w) * D + lane * E + e] = x[e];
+    sx[r][lane * E + e] = x[e];
     hi = max(hi, (uint32_t)__double2hiint(x[e]) & 0x7fffffffu);
     const float xw = (float)x[e] * (float)(D - (lane * E + e) + kEvalUlps);
     ss = fmaf(xw, xw, ss);
@@ -158,24 +184,34 @@ __global__ __launch_bounds__(256) void qdigit_kernel(const T* __restrict__ q, co
     u[e] = ((uint32_t)v + kBalance) ^ kBalance;
   }
   const int d = lane * E, t = d >> 5;
-  int8_t* dst = qd + row * D * kDigits +
-                ((int64_t)(w >> 4) * kDigits * (D / 64) + (t >> 1)) * 1024 + (((d >> 3) & 3) * 16 + (w & 15)) * 16 +
-                (t & 1) * 8 + (d & 7);
+  // sd: [digit][k-step][kk][row of 4][16]
+  int8_t* dst = reinterpret_cast<int8_t*>(sd) + (t >> 1) * 256 + (((d >> 3) & 3) * 4 + r) * 16 + (t & 1) * 8 + (d & 7);
 #pragma unroll
   for (int j = 0; j < kDigits; ++j)
 #pragma unroll
-    for (int e = 0; e < E; ++e) dst[(int64_t)j * (D / 64) * 1024 + e] = (int8_t)(u[e] >> (8 * j));
+    for (int e = 0; e < E; ++e) dst[j * (D / 64) * 256 + e] = (int8_t)(u[e] >> (8 * j));
   ss = __uint_as_float(reduce_cols(reduce_rows(__float_as_uint(ss), SumF32{}), SumF32{}));
   res = __uint_as_float(reduce_cols(reduce_rows(__float_as_uint(res), SumF32{}), SumF32{}));
   if (lane == 0) {
     // rounded up, past what the fp32 sums lose, to underflow too
     const float up = 1.f + 0x1p-14f, tiny = 1e-17f;
-    QDigitRow r;
-    r.scale = use ? ldexp(1.0, -sh) : 1.0;
-    r.norm = hi == 0 || use ? sqrtf(ss) * up + tiny : INFINITY;
-    r.resid = res * up + 2e-36f;
-    qrow[row + w] = r;
+    QDigitRow o;
+    o.scale = use ? ldexp(1.0, -sh) : 1.0;
+    o.norm = hi == 0 || use ? sqrtf(ss) * up + tiny : INFINITY;
+    o.resid = res * up + 2e-36f;
+    qrow[row + w] = o;
   }
+  __syncthreads();
+  const int64_t at = (row + (w >> 4) * 16) * D;      // the row block
+  const int r0 = (int)blockIdx.x % 4 * 4;
+  doublex2* of = reinterpret_cast<doublex2*>(qf + at);
+  i32x4* od = reinterpret_cast<i32x4*>(qd + at * kDigits);
+#pragma unroll
+  for (int i = tid; i < 2 * D; i += 256) {           // piece i: dims 8 (i / 16) + (i / 4) % 4, row i % 4
+    const int c = (i >> 4) * 8 + ((i >> 2) & 3);
+    of[(i >> 2) * 16 + r0 + (i & 3)] = doublex2{sx[i & 3][c], sx[i & 3][c + 4]};
+  }
+  if (tid < D * kDigits / 4) od[(tid >> 2) * 16 + r0 + (tid & 3)] = sd[tid];
 }
 
 // Fixed point of key rows: |x| * 2^(kShift - f) <= kFixMax for every element,
@@ -212,10 +248,12 @@ struct KDigits {
   static constexpr int NP = D / 32;   // 16-byte pieces per lane
   static constexpr int NS = D / 64;   // k-steps
   i32x4 d[kDigits][NS];
-  int f;        // scale 2^(f - kShift)
-  float norm;   // +inf if an element is not held exactly
+  i32x4 low[NS];   // the fifth digit, of weight 2^-8
+  int f;           // scale 2^(f - kShift)
+  int held;        // digits that hold every element exactly: 4, 5, or 0 if no five do
+  float norm;
 
-  __device__ __forceinline__ void convert(const uint32_t (&w)[NP][4]) {
+  __device__ __forceinline__ void scan(const uint32_t (&w)[NP][4]) {
     using F = KFix<T>;
     u16x2 mx = {0, 0};
     float ss = 0.f;
@@ -230,7 +268,7 @@ struct KDigits {
     const int mb = __builtin_amdgcn_readfirstlane((int)max(hi & 0xffffu, hi >> 16));
     // a mantissa at 2 - 2^-7 or above would pass kFixMax
     f = max((mb + (1 << (F::kMant - 7))) >> F::kMant, F::kMinF);
-    bool exact = mb < F::kInf;
+    held = kDigits;
     if (f > F::kExactF) {       // wave-uniform: the smallest non-zero element decides
       u16x2 mn = {0xffff, 0xffff};
 #pragma unroll
@@ -241,18 +279,40 @@ struct KDigits {
           mn = __builtin_elementwise_min(mn, (u16x2)(a - (u16x2){1, 1}));   // zeros wrap to 0xffff
         }
       const uint32_t lo = reduce_cols(reduce_rows(~__builtin_bit_cast(uint32_t, mn), MaxU16x2{}), MaxU16x2{});
-      const int nb = 0x10000 - (int)max(lo & 0xffffu, lo >> 16);
-      exact = exact && max(nb >> F::kMant, 1) >= f - (30 - F::kMant);
+      const int nb = __builtin_amdgcn_readfirstlane(0x10000 - (int)max(lo & 0xffffu, lo >> 16));
+      const int below = f - (30 - F::kMant) - max(nb >> F::kMant, 1);   // bits below the four digits
+      held = below <= 0 ? 4 : below <= 8 ? 5 : 0;
     }
+    if (mb >= F::kInf) held = 0;
+    // An fp32 sum of D squares and its root: within 2^-14.  Half subnormals,
+    // which the dot product may take as zero, are below sqrt(D) * 2^-14.
+    ss = __uint_as_float(reduce_cols(reduce_rows(__float_as_uint(ss), SumF32{}), MaxF32{}));
+    norm = sqrtf(ss) * (1.f + 0x1p-14f) + 0x1p-10f;
+  }
+
+  // With LOW the four digits hold the nearest integer and the fifth the rest.
+  template <bool LOW>
+  __device__ __forceinline__ void digits(const uint32_t (&w)[NP][4]) {
+    using F = KFix<T>;
     const float mult = __uint_as_float((uint32_t)(127 + F::kShift - f) << 23);
 #pragma unroll
     for (int p = 0; p < NP; ++p)
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
-        uint32_t u[4];
+        uint32_t u[4], rest = 0;
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
-          u[i] = (uint32_t)(int)__builtin_fmaf(F::get(w[p][2 * h + (i >> 1)], i & 1), mult, 0.f) + kBalance;
+        for (int i = 0; i < 4; ++i) {
+          const float x = F::get(w[p][2 * h + (i >> 1)], i & 1);
+          float v = __builtin_fmaf(x, mult, 0.f);
+          if constexpr (LOW) {
+            // the nearest integer (a fraction needs |v| < 2^11, so v + 1/2 is
+            // exact where it matters) and 256ths of the rest, plus 128
+            const float n = __builtin_floorf(v + 0.5f);
+            rest = __builtin_amdgcn_cvt_pk_u8_f32(__builtin_fmaf(v - n, 256.f, 128.f), i, rest);
+            v = n;
+          }
+          u[i] = (uint32_t)(int)v + kBalance;
+        }
         // bytes of the four elements regrouped by digit
         const uint32_t a0 = __builtin_amdgcn_perm(u[1], u[0], 0x05010400u);
         const uint32_t a1 = __builtin_amdgcn_perm(u[1], u[0], 0x07030602u);
@@ -263,54 +323,101 @@ struct KDigits {
         d[1][p >> 1][at] = (int)(__builtin_amdgcn_perm(b0, a0, 0x07060302u) ^ kBalance);
         d[2][p >> 1][at] = (int)(__builtin_amdgcn_perm(b1, a1, 0x05040100u) ^ kBalance);
         d[3][p >> 1][at] = (int)(__builtin_amdgcn_perm(b1, a1, 0x07060302u) ^ kBalance);
+        if constexpr (LOW) low[p >> 1][at] = (int)(rest ^ kBalance);
       }
-    // An fp32 sum of D squares and its root: within 2^-14.  Half subnormals,
-    // which the dot product may take as zero, are below sqrt(D) * 2^-14.
-    ss = __uint_as_float(reduce_cols(reduce_rows(__float_as_uint(ss), SumF32{}), MaxF32{}));
-    const float n = sqrtf(ss) * (1.f + 0x1p-14f) + 0x1p-10f;
-    norm = exact ? n : INFINITY;
   }
 };
 
-// One 16-key x 16-row tile by the defining fp64 chain (keys key0.., rows wt..
-// of the workgroup's block at window row w0; qf at the tile's first row):
-// stores its logits and folds its row maxima into redk.
-template <typename T, int MODE, int D>
-__device__ __forceinline__ void redo_tile(__amdgpu_buffer_rsrc_t krs, uint32_t rowb, const double* qf,
-                                       __amdgpu_buffer_rsrc_t lrs, int S, int ld, int key0, int w0, int wt, int nw,
-                                       int qpos0, double scaling, uint32_t* redk) {
+// NB 16-key x 16-row tiles by the defining fp64 chain: the keys key0.. that the
+// wave holds in w (as the logits kernel loads them), rows wt.. of the
+// workgroup's block at window row w0.  Stores the logits and folds the lane's
+// maxima of rows wt + 16 t + kk + 4 i into top[t][i].  fetch(row block, pair of
+// k-steps) gives a lane its two queries; AHEAD pairs of them are under way.  The
+// matrix unit's fp64 products hide few vector instructions, so there are few:
+// the addresses are scalar offsets.
+template <typename T, int MODE, int D, int NB, int AHEAD, typename F>
+__device__ __forceinline__ void chain_tiles(const uint32_t (&w)[D / 32][4], F&& fetch, __amdgpu_buffer_rsrc_t lrs,
+                                            int ld, int key0, int w0, int wt, int nw, int qpos0, double scaling,
+                                            float (&top)[NB][4]) {
   typedef double doublex4 __attribute__((ext_vector_type(4)));
-  const int lane = threadIdx.x & 63, col = lane & 15, kk = lane >> 4;
-  const uint32_t koff = key0 + col < S ? (uint32_t)(key0 + col) * rowb + 2u * kk : kOob;
-  const double* qr = qf + col * D + kk;   // zero rows past the window
-  const int w = wt + col;
-  doublex4 acc = {0.0, 0.0, 0.0, 0.0};
-  // every operand in flight at once: in four batches the loads' round trips
-  // were most of the tile's time (with the tighter norm of QDigitRow 4% of the
-  // f16 launches' time and 10% of the bf16 one's)
-  uint32_t kw[D / 4];
-  double q[D / 4];
+  constexpr int NU = D / 8;
+  int lane = threadIdx.x & 63;
+  // what follows from the lane is worked out here: hoisted out of the caller's
+  // chunk loop, it would hold registers (or scratch) in the common path too
+  __asm__ volatile("" : "+v"(lane));
+  const int col = lane & 15, kk = lane >> 4, key = key0 + col;
+  doublex4 acc[NB];
+  doublex2 q[AHEAD][NB];
 #pragma unroll
-  for (int t = 0; t < D / 4; ++t) {
-    kw[t] = __builtin_amdgcn_raw_buffer_load_b16(krs, (int)koff, t * 8, 0);
-    q[t] = qr[t * 4];
+  for (int i = 0; i < NB; ++i) acc[i] = doublex4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+  for (int u = 0; u < AHEAD; ++u)
+#pragma unroll
+    for (int i = 0; i < NB; ++i) q[u][i] = fetch(i, u);
+  static_assert(4 % AHEAD == 0, "whole turns of the ring in a piece");
+#pragma unroll
+  for (int u0 = 0; u0 < NU; u0 += 4) {
+    const uint32_t(&wp)[4] = w[u0 / 4];
+    // A lane holds 8 consecutive dims of its key, the key's four lanes 32; a
+    // k-step wants dim 4t + kk in lane kk.  Dims kk and kk + 4 of a lane are
+    // packed for lane kk, and the four packed words go their ways as a 4 x 4
+    // transpose over the rows of 16 lanes: x[g] then holds lane kk's dims of
+    // k-steps 2 (u0 + g) and 2 (u0 + g) + 1.
+    uint32_t x[4];
+    x[0] = __builtin_amdgcn_perm(wp[2], wp[0], 0x05040100u);
+    x[1] = __builtin_amdgcn_perm(wp[2], wp[0], 0x07060302u);
+    x[2] = __builtin_amdgcn_perm(wp[3], wp[1], 0x05040100u);
+    x[3] = __builtin_amdgcn_perm(wp[3], wp[1], 0x07060302u);
+#pragma unroll
+    for (int i = 0; i < 4; i += 2) {
+      const auto s = __builtin_amdgcn_permlane16_swap(x[i], x[i + 1], false, false);
+      x[i] = s[0];
+      x[i + 1] = s[1];
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const auto s = __builtin_amdgcn_permlane32_swap(x[i], x[i + 2], false, false);
+      x[i] = s[0];
+      x[i + 2] = s[1];
+    }
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+        const double kd = (double)KFix<T>::get(x[g], s);
+#pragma unroll
+        for (int i = 0; i < NB; ++i)
+          acc[i] = __builtin_amdgcn_mfma_f64_16x16x4f64(q[g % AHEAD][i][s], kd, acc[i], 0, 0, 0);
+      }
+      if (u0 + g + AHEAD < NU)
+#pragma unroll
+        for (int i = 0; i < NB; ++i) q[g % AHEAD][i] = fetch(i, u0 + g + AHEAD);
+    }
   }
+  // Lane (kk, col): rows kk + 4i of the tiles, key col.
+  const uint32_t off = key < ld ? (uint32_t)((w0 + wt + kk) * ld + key) * 4u : kOob;
+  auto finish = [&](auto plain_c) {
+    constexpr bool PLAIN = decltype(plain_c)::value;
 #pragma unroll
-  for (int t = 0; t < D / 4; ++t)
-    acc = __builtin_amdgcn_mfma_f64_16x16x4f64((double)KFix<T>::get(kw[t], 0), q[t], acc, 0, 0, 0);
-  float m = -INFINITY;
+    for (int t = 0; t < NB; ++t)
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {   // keys kk + 4i, row col
-    const int key = key0 + kk + 4 * i;
-    float L;
-    if constexpr (MODE == HC_SCORE_SNAPKV) L = key > qpos0 + w ? -INFINITY : (float)(acc[i] * scaling);
-    else L = (float)(acc[i] / scaling);
-    const bool ok = key < ld && w < nw;
-    const uint32_t bits = __float_as_uint(L);
-    bstore<4>(lrs, ok ? (uint32_t)((w0 + w) * ld + key) * 4u : kOob, &bits);
-    m = fmaxf(m, ok ? L : -INFINITY);
-  }
-  if (w < nw) atomicMax(&redk[w], order_key(m));
+      for (int i = 0; i < 4; ++i) {
+        const int r = 16 * t + 4 * i;
+        float L;
+        if constexpr (MODE == HC_SCORE_SNAPKV) L = (float)(acc[t][i] * scaling);
+        else L = (float)(acc[t][i] / scaling);
+        uint32_t o = off;
+        if constexpr (!PLAIN) {
+          if constexpr (MODE == HC_SCORE_SNAPKV) L = key > qpos0 + wt + kk + r ? -INFINITY : L;
+          o = wt + kk + r < nw ? off : kOob;
+        }
+        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(L), lrs, (int)o, (int)((uint32_t)(r * ld) * 4u), 0);
+        if constexpr (MODE == HC_SCORE_SNAPKV) top[t][i] = fmaxf(top[t][i], L);
+      }
+  };
+  // wave-uniform: every key at or before every row's position, every row real
+  if ((MODE != HC_SCORE_SNAPKV || key0 + 15 <= qpos0 + wt) && wt + 16 * NB <= nw) finish(std::true_type{});
+  else finish(std::false_type{});
 }
 
 // The logits kernel.  grid (ceil(S / (64 * cpw)), Hk * ceil(W / (16 * NRB)),
@@ -319,7 +426,11 @@ __device__ __forceinline__ void redo_tile(__amdgpu_buffer_rsrc_t krs, uint32_t r
 // in registers while the row blocks' digits come from LDS, 16 rows at a time.
 // Keys are the A operand, so a lane's four results are consecutive keys of one
 // row: one 16-byte store.  The next chunk's keys are loaded while this one is
-// multiplied.
+// multiplied.  Chunks that take more than four digits are left for two loops of
+// their own, the chain's with the queries in LDS for the whole workgroup: each
+// form keeps its registers, and the chain's tiles their matrix rate (the same
+// tiles redone one by one in place, the queries read from memory, took five
+// times the fp64 kernel).
 template <typename T, int MODE, int D, int NRB>
 __global__ __launch_bounds__(256, 3) void logits_i8_kernel(
     const T* __restrict__ k, const T* const* __restrict__ k_rows, int64_t k_sb, int64_t k_sh, int64_t k_ss,
@@ -327,10 +438,14 @@ __global__ __launch_bounds__(256, 3) void logits_i8_kernel(
     const QDigitRow* __restrict__ qrow, int Hk, int S, int W, int wpad, double scaling, int cpw, int ld,
     float* __restrict__ logits, uint32_t* __restrict__ rmax) {
   constexpr int ROWS = 16 * NRB, NS = D / 64, NP = D / 32, CHUNK = kDigitChunk;
-  __shared__ i32x4 sq[NRB * kDigits * NS * 64];
+  constexpr int PB = NRB < 2 ? NRB : 2;       // row blocks per pass over the hard chunks
+  constexpr int SQ_DIGITS = NRB * kDigits * NS * 64, SQ_CHAIN = PB * 8 * D;
+  __shared__ i32x4 sq[SQ_DIGITS > SQ_CHAIN ? SQ_DIGITS : SQ_CHAIN];
   __shared__ double ssc[ROWS];       // row scale times the logit scale
-  __shared__ double sdel[NRB];       // a key of 2-norm 1's delta against the row block
+  __shared__ double sdel[ROWS];      // a key of 2-norm 1's delta against the row
   __shared__ uint32_t redk[ROWS];
+  __shared__ int open_s;             // the rows' residuals leave most tiles open
+  __shared__ int hard_s;             // a wave has hard chunks
   const int nrb = (W + ROWS - 1) / ROWS, nx = (int)gridDim.x;
   const int fl = (int)blockIdx.x + nx * (int)blockIdx.y;
   const int rb = nrb - 1 - fl % nrb;
@@ -354,14 +469,16 @@ __global__ __launch_bounds__(256, 3) void logits_i8_kernel(
 
   int key0 = wg_key0 + wave * 16;
   uint32_t raw[NP][4];
-  auto load = [&](int at) {
+  auto load_keys = [&](uint32_t (&dst)[NP][4], int at) {
     const int key = at + col;
     const uint32_t off = key < S ? (uint32_t)key * rowb + 16u * kk : kOob;
 #pragma unroll
-    for (int p = 0; p < NP; ++p) bload_so<16>(krs, off, 64u * p, raw[p]);
+    for (int p = 0; p < NP; ++p) bload_so<16>(krs, off, 64u * p, dst[p]);
   };
+  auto load = [&](int at) { load_keys(raw, at); };
   load(key0);
   if (tid < ROWS) redk[tid] = order_key(-INFINITY);
+  if (tid == 0) open_s = hard_s = 0;
   if (stage) {
     const i32x4* src = reinterpret_cast<const i32x4*>(qd + (bh * wpad + w0) * (int64_t)(D * kDigits));
 #pragma unroll
@@ -370,13 +487,16 @@ __global__ __launch_bounds__(256, 3) void logits_i8_kernel(
     if (tid < ROWS) {
       const QDigitRow r = qrow[bh * wpad + w0 + tid];
       ssc[tid] = r.scale * lscale;
-      double dl = (double)r.norm * 0x1p-53 + (double)r.resid;
+      sdel[tid] = ((double)r.norm * 0x1p-53 + (double)r.resid) * fabs(lscale) * 1.001;
+      float open = r.norm < INFINITY ? r.resid / r.norm : INFINITY;
 #pragma unroll
-      for (int o = 8; o > 0; o >>= 1) dl = fmax(dl, __shfl_xor(dl, o, 64));
-      if (col == 0) sdel[tid >> 4] = dl * fabs(lscale) * 1.001;
+      for (int o = ROWS / 2; o > 0; o >>= 1) open += __shfl_xor(open, o, 64);
+      if (tid == 0) open_s = open > NRB * kOpenRatio;
     }
   }
   __syncthreads();
+  const bool open_rows = __builtin_amdgcn_readfirstlane(open_s);
+  const double* qrows = qf + (bh * wpad + w0) * D;
 
   const int nch = key0 < S ? min(cpw, (S - key0 + CHUNK - 1) / CHUNK) : 0;
   int nmul = nch;
@@ -387,107 +507,218 @@ __global__ __launch_bounds__(256, 3) void logits_i8_kernel(
   float mrow[NRB];
 #pragma unroll
   for (int i = 0; i < NRB; ++i) mrow[i] = -INFINITY;
+  // chain_tiles' maxima of rows wt .. into redk
+  auto fold = [&](const auto& top, int wt) {
+    if constexpr (MODE == HC_SCORE_SNAPKV)
+#pragma unroll
+      for (int t = 0; t < (int)(sizeof(top) / sizeof(top[0])); ++t)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) atomicMax(&redk[wt + 16 * t + kk + 4 * i], order_key(top[t][i]));
+  };
 
-  for (int c = 0; c < nmul; ++c) {
-    // the row blocks' LDS reads repeat for every chunk: hoisted, they would
-    // hold registers for the kernel's lifetime
-    __asm__ volatile("" ::: "memory");
-    KDigits<T, D> kd;
-    kd.convert(raw);
-    load(key0 + CHUNK);
-    // every key at or before every row's position, none past S
-    const bool plain = key0 + 16 <= S && (MODE != HC_SCORE_SNAPKV || key0 + 16 - 1 <= qpos0);
-    uint32_t redo = 0;
-    // The products of row block nb against the chunk's keys.
-    auto multiply = [&](i32x4 (&acc)[2 * kDigits - 1], int nb) {
+  // The products of row block nb against the chunk's keys; with LOW the fifth
+  // digits' too, rest of weight 2^-8.
+  auto multiply = [&](const KDigits<T, D>& kd, i32x4 (&acc)[2 * kDigits - 1], i32x4& rest, int nb, auto low_c) {
 #pragma unroll
-      for (int j = 0; j < kDigits; ++j) {
-        i32x4 q[NS];
+    for (int j = 0; j < kDigits; ++j) {
+      i32x4 q[NS];
 #pragma unroll
-        for (int s = 0; s < NS; ++s) q[s] = sq[((nb * kDigits + j) * NS + s) * 64 + lane];
+      for (int s = 0; s < NS; ++s) q[s] = sq[((nb * kDigits + j) * NS + s) * 64 + lane];
 #pragma unroll
-        for (int s = 0; s < NS; ++s)
+      for (int s = 0; s < NS; ++s)
 #pragma unroll
-          for (int i = 0; i < kDigits; ++i) {
-            const bool first = s == 0 && (j == 0 || i == kDigits - 1);   // of its weight
-            acc[i + j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(kd.d[i][s], q[s],
-                                                               first ? i32x4{0, 0, 0, 0} : acc[i + j], 0, 0, 0);
+        for (int i = 0; i < kDigits; ++i) {
+          const bool first = s == 0 && (j == 0 || i == kDigits - 1);   // of its weight
+          acc[i + j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(kd.d[i][s], q[s],
+                                                             first ? i32x4{0, 0, 0, 0} : acc[i + j], 0, 0, 0);
+        }
+      if constexpr (decltype(low_c)::value)
+#pragma unroll
+        for (int s = 0; s < NS; ++s) {
+          i32x4& to = j ? acc[j - 1] : rest;
+          to = __builtin_amdgcn_mfma_i32_16x16x64_i8(kd.low[s], q[s], j + s ? to : i32x4{0, 0, 0, 0}, 0, 0, 0);
+        }
+    }
+  };
+  // Their logits: stored, or the tile marked for the fp64 chain.  PLAIN: no row
+  // before a key's position, no key past the last or all zero (its logits are
+  // 0: with a delta of more they would all be redone).
+  auto finish = [&](const KDigits<T, D>& kd, const i32x4 (&acc)[2 * kDigits - 1], const i32x4& rest, int key0,
+                    uint32_t& redo, int nb, auto plain_c, auto low_c) {
+    constexpr bool PLAIN = decltype(plain_c)::value, LOW = decltype(low_c)::value;
+    const int w = 16 * nb + col;
+    const double rs = ssc[w], dl = sdel[w];
+    const uint64_t live = ((1ull << min(max(nw - 16 * nb, 0), 16)) - 1) * 0x0001000100010001ull;   // real rows' lanes
+    const double del = dl * (double)kd.norm;
+    const double sc = rs * __hiloint2double((1023 + kd.f - KFix<T>::kShift) << 20, 0);
+    const int key = key0 + 4 * kk;
+    float L[4];
+    bool open = false;       // a logit that delta does not settle
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int t0 = (acc[6][i] << 8) + acc[5][i];
+      const int t1 = (acc[4][i] << 8) + acc[3][i];
+      const int t2 = (acc[2][i] << 8) + acc[1][i];
+      double d = __builtin_fma(__builtin_fma(__builtin_fma((double)t0, 65536.0, (double)t1), 65536.0,
+                                             (double)t2), 256.0, (double)acc[0][i]);
+      if constexpr (LOW) d = __builtin_fma((double)rest[i], 0x1p-8, d);
+      const float lo = (float)__builtin_fma(d, sc, -del);
+      L[i] = (float)__builtin_fma(d, sc, del);
+      bool bad = !(lo == L[i]);
+      if constexpr (!PLAIN) {
+        if constexpr (MODE == HC_SCORE_SNAPKV)
+          if (key + i > qpos0 + w) {
+            L[i] = -INFINITY;
+            bad = false;
           }
+        bad = bad && key + i < S;
       }
-    };
-    // Their logits: stored, or the tile marked for redo_tile.
-    auto finish = [&](const i32x4 (&acc)[2 * kDigits - 1], int nb, auto plain_c) {
-      constexpr bool PLAIN = decltype(plain_c)::value;
-      const int w = 16 * nb + col;
-      const double rs = ssc[w], dl = sdel[nb];
-      const uint64_t live = ((1ull << min(max(nw - 16 * nb, 0), 16)) - 1) * 0x0001000100010001ull;   // real rows' lanes
-      const double del = dl * (double)kd.norm;
-      const double sc = rs * __hiloint2double((1023 + kd.f - KFix<T>::kShift) << 20, 0);
-      const int key = key0 + 4 * kk;
-      float L[4];
-      bool open = false;       // a logit that delta does not settle
+      open |= bad;
+    }
+    // The stores are issued either way (out of range for an open tile): the
+    // wait for the next chunk's keys counts them, and behind a branch it
+    // would have to wait for the stores too.
+    const bool again = (__ballot(open) & live) != 0;    // wave-uniform
+    redo |= again ? 1u << nb : 0u;
+    const bool ok = w < nw && !again;
+    const uint32_t off = ok ? (uint32_t)((w0 + w) * ld + key) * 4u : kOob;
+    const uint32_t bits[4] = {__float_as_uint(L[0]), __float_as_uint(L[1]), __float_as_uint(L[2]),
+                              __float_as_uint(L[3])};
+    if constexpr (PLAIN) {
+      bstore<16>(lrs, off, bits);
+      if constexpr (MODE == HC_SCORE_SNAPKV)
+        mrow[nb] = fmaxf(mrow[nb], ok ? fmaxf(fmaxf(L[0], L[1]), fmaxf(L[2], L[3])) : -INFINITY);
+    } else {
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const int t0 = (acc[6][i] << 8) + acc[5][i];
-        const int t1 = (acc[4][i] << 8) + acc[3][i];
-        const int t2 = (acc[2][i] << 8) + acc[1][i];
-        const double d = __builtin_fma(__builtin_fma(__builtin_fma((double)t0, 65536.0, (double)t1), 65536.0,
-                                                     (double)t2), 256.0, (double)acc[0][i]);
-        const float lo = (float)__builtin_fma(d, sc, -del);
-        L[i] = (float)__builtin_fma(d, sc, del);
-        bool bad = !(lo == L[i]);
-        if constexpr (!PLAIN) {
-          if constexpr (MODE == HC_SCORE_SNAPKV)
-            if (key + i > qpos0 + w) {
-              L[i] = -INFINITY;
-              bad = false;
-            }
-          bad = bad && key + i < S;
-        }
-        open |= bad;
+        bstore<4>(lrs, key + i < ld ? off + 4u * i : kOob, &bits[i]);   // kOob + 12 is out of range too
+        if constexpr (MODE == HC_SCORE_SNAPKV) mrow[nb] = fmaxf(mrow[nb], ok && key + i < S ? L[i] : -INFINITY);
       }
-      // The stores are issued either way (out of range for an open tile): the
-      // wait for the next chunk's keys counts them, and behind a branch it
-      // would have to wait for the stores too.
-      const bool again = (__ballot(open) & live) != 0;    // wave-uniform
-      redo |= again ? 1u << nb : 0u;
-      const bool ok = w < nw && !again;
-      const uint32_t off = ok ? (uint32_t)((w0 + w) * ld + key) * 4u : kOob;
-      const uint32_t bits[4] = {__float_as_uint(L[0]), __float_as_uint(L[1]), __float_as_uint(L[2]),
-                                __float_as_uint(L[3])};
-      if constexpr (PLAIN) {
-        bstore<16>(lrs, off, bits);
-        if constexpr (MODE == HC_SCORE_SNAPKV)
-          mrow[nb] = fmaxf(mrow[nb], ok ? fmaxf(fmaxf(L[0], L[1]), fmaxf(L[2], L[3])) : -INFINITY);
-      } else {
+    }
+  };
+  auto row_blocks = [&](const KDigits<T, D>& kd, int key0, auto plain_c, auto low_c) {
+    uint32_t redo = 0;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          bstore<4>(lrs, key + i < ld ? off + 4u * i : kOob, &bits[i]);   // kOob + 12 is out of range too
-          if constexpr (MODE == HC_SCORE_SNAPKV) mrow[nb] = fmaxf(mrow[nb], ok && key + i < S ? L[i] : -INFINITY);
-        }
-      }
-    };
-    auto row_blocks = [&](auto plain_c) {
-#pragma unroll
-      for (int nb = 0; nb < NRB; ++nb) {
-        i32x4 acc[2 * kDigits - 1];
-        multiply(acc, nb);
-        finish(acc, nb, plain_c);
-      }
-    };
-    // compiled apart, so that the common form is straight-line code
-    if (plain) row_blocks(std::true_type{});
-    else row_blocks(std::false_type{});
-    while (redo) {               // wave-uniform
+    for (int nb = 0; nb < NRB; ++nb) {
+      i32x4 acc[2 * kDigits - 1], rest;
+      multiply(kd, acc, rest, nb, low_c);
+      finish(kd, acc, rest, key0, redo, nb, plain_c, low_c);
+      // side by side, two row blocks with a fifth digit would need more
+      // registers than the common form
+      if constexpr (decltype(low_c)::value) __builtin_amdgcn_sched_barrier(0);
+    }
+    return redo;
+  };
+  auto redo_tiles = [&](uint32_t redo, int key0) {
+    if (!redo) return;           // wave-uniform
+    uint32_t cur[NP][4];
+    load_keys(cur, key0);
+    while (redo) {
       const int nb = __ffs(redo) - 1;
       redo &= redo - 1;
-      redo_tile<T, MODE, D>(krs, rowb, qf + (bh * wpad + w0 + 16 * nb) * D, lrs, S, ld, key0, w0,
-                            16 * nb, nw, qpos0, scaling, redk);
+      const __amdgpu_buffer_rsrc_t qrs = make_rsrc(qrows + 16 * nb * D, 16 * D * 8);
+      float top[1][4] = {{-INFINITY, -INFINITY, -INFINITY, -INFINITY}};
+      chain_tiles<T, MODE, D, 1, 4>(cur, [&](int, int u) {
+        uint32_t r[4];
+        bload_so<16>(qrs, 16u * lane, 1024u * u, r);
+        return __builtin_bit_cast(doublex2, u32x4{r[0], r[1], r[2], r[3]});
+      }, lrs, ld, key0, w0, 16 * nb, nw, qpos0, scaling, top);
+      fold(top, 16 * nb);
     }
-    key0 += CHUNK;
+  };
+  auto chunk = [&](int c) { return wg_key0 + wave * 16 + c * CHUNK; };
+
+  // Chunks whose keys need a fifth digit, and those that only the fp64 chain
+  // does, are left for the loops below (bit c of wide and hard).  After two at
+  // the start the rest is left unseen: where all are, looking costs a read of
+  // the keys.  `in` is the chunk that raw holds.
+  const uint32_t all = (1u << nmul) - 1;
+  uint32_t wide = 0, hard = open_rows ? all : 0;
+  int in = 0;
+  if (!open_rows)
+    for (int c = 0; c < nmul; ++c) {
+      // the row blocks' LDS reads repeat for every chunk: hoisted, they would
+      // hold registers for the kernel's lifetime
+      __asm__ volatile("" ::: "memory");
+      KDigits<T, D> kd;
+      kd.scan(raw);
+      if (kd.held != kDigits) {    // wave-uniform
+        wide |= 1u << c;
+        if (wide == 3) wide = all;
+        in = c;
+        if (c + 1 == nmul || wide == all) break;
+        load(key0 + CHUNK);
+        key0 += CHUNK;
+        continue;
+      }
+      kd.template digits<false>(raw);
+      load(key0 + CHUNK);
+      in = c + 1;
+      const bool plain = key0 + 16 <= S && (MODE != HC_SCORE_SNAPKV || key0 + 16 - 1 <= qpos0);
+      // compiled apart, so that the common form is straight-line code
+      redo_tiles(plain ? row_blocks(kd, key0, std::true_type{}, std::false_type{})
+                       : row_blocks(kd, key0, std::false_type{}, std::false_type{}), key0);
+      key0 += CHUNK;
+    }
+  // last first: it may be in
+  for (uint32_t left = wide; left;) {
+    __asm__ volatile("" ::: "memory");
+    const int c = 31 - __clz(left), at = chunk(c);
+    left &= ~(1u << c);
+    // (not loaded ahead: the fifth digit takes the registers)
+    if (in != c) load(at);
+    in = c;
+    KDigits<T, D> kd;
+    kd.scan(raw);
+    if (kd.held) {               // wave-uniform
+      kd.template digits<true>(raw);
+      redo_tiles(row_blocks(kd, at, std::false_type{}, std::true_type{}), at);
+      continue;
+    }
+    hard |= 1u << c;
+    if (__popc(hard) == 2 && hard == (wide & ~left)) {
+      hard = wide;
+      break;
+    }
+  }
+
+  // The hard chunks, PB row blocks' queries in LDS at a time (in place of the
+  // digits).
+  if (hard && lane == 0) hard_s = 1;
+  __syncthreads();
+  if (hard_s) {                  // workgroup-uniform
+    const doublex2* sx = reinterpret_cast<const doublex2*>(sq);
+    for (int wt = 0; wt < nw; wt += 16 * PB) {
+      const i32x4* src = reinterpret_cast<const i32x4*>(qrows + wt * D);
+      for (int i = tid; i < SQ_CHAIN; i += 256) sq[i] = src[i];
+      __syncthreads();
+      uint32_t left = hard;
+      float top[PB][4];
+#pragma unroll
+      for (int t = 0; t < PB; ++t)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) top[t][i] = -INFINITY;
+      if (left && __ffs(left) - 1 != in) load(chunk(__ffs(left) - 1));
+      in = -1;
+      while (left) {             // wave-uniform
+        const int at = chunk(__ffs(left) - 1);
+        left &= left - 1;
+        uint32_t cur[NP][4];
+#pragma unroll
+        for (int p = 0; p < NP; ++p)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) cur[p][i] = raw[p][i];
+        if (left) load(chunk(__ffs(left) - 1));
+        chain_tiles<T, MODE, D, PB, 2>(cur, [&](int i, int u) { return sx[(i * (D / 8) + u) * 64 + lane]; }, lrs, ld,
+                                       at, w0, wt, nw, qpos0, scaling, top);
+      }
+      if (hard) fold(top, wt);
+      __syncthreads();
+    }
   }
 
   if constexpr (MODE != HC_SCORE_SNAPKV) return;
+  key0 = chunk(nmul);
   for (int c = nmul; c < nch && key0 <= qpos0 + nw - 1 + kNeverRead; ++c) {   // wholly masked chunks
     const uint32_t ninf = __float_as_uint(-INFINITY);
 #pragma unroll

@@ -591,6 +591,9 @@ def _digit_inputs(kind, shape_q, shape_k, dtype):
     g = torch.Generator().manual_seed(83)
     if kind == "outliers":
         k[..., :3] *= 40.0
+    elif kind == "mixed":         # runs of keys for four digits, five, and none at all
+        runs = torch.tensor([1.0, 300.0, 1e4, 1e9]).repeat_interleave(50)
+        k[..., 1] = (k[..., 1] * runs.repeat(k.shape[2] // 200 + 1)[:k.shape[2]]).clamp(-6e4, 6e4)
     elif kind == "wide":
         q, k = (t * torch.exp2(torch.randint(-12, 13, t.shape, generator=g).float()) for t in (q, k))
     elif kind == "tiny":
@@ -617,7 +620,8 @@ def _digit_inputs(kind, shape_q, shape_k, dtype):
 
 @pytest.mark.parametrize("W,S,D", [(1, 200, 128), (8, 331, 64), (17, 1027, 128), (33, 517, 64), (65, 1100, 128)])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
-@pytest.mark.parametrize("kind", ["normal", "outliers", "wide", "tiny", "huge", "zeros", "ends", "cancel", "special"])
+@pytest.mark.parametrize("kind", ["normal", "outliers", "mixed", "wide", "tiny", "huge", "zeros", "ends", "cancel",
+                                  "special"])
 def test_window_logits_digits_equal_fp64_chain(kind, dtype, W, S, D):
     """Groups of three equal query heads have the mean of one of them, bit for
     bit, and run on the fp64 kernel; groups of one and two run on the digits."""
@@ -651,6 +655,34 @@ def test_long_window_scores_bit_exact(W, S, dtype, pool):
     want = ref.window_scores(q, k, W, 0.125, pool, "avgpool")
     assert torch.isnan(got[:, 0]).all() and torch.equal(got.isnan(), want.isnan())
     assert torch.equal(got.nan_to_num(), want.nan_to_num())
+
+
+@pytest.mark.parametrize("kind", ["query", "wide400", "beyond", "all"])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("W,D,Hq", [(16, 64, 8), (32, 128, 8), (64, 128, 16), (50, 64, 8)])
+def test_window_logits_of_every_digit_form_over_many_chunks(kind, dtype, W, D, Hq):
+    """Workgroups of several 64-key chunks whose keys take four digits, five
+    and the fp64 chain by turns, or one of them throughout, with queries that
+    have digits and with some that leave most tiles open: the scores are those
+    of groups of three equal heads, which run on the fp64 kernel."""
+    B, Hk, S = 6, 8, 64 * 250 + 13 if Hq == 8 else 64 * 120 + 13
+    q, k = _randn((B, Hk, S, D), 95, torch.float32), _randn((B, Hk, S, D), 96, torch.float32)
+    runs = torch.arange(S) // 48 % 5
+    if kind in ("wide400", "all"):
+        k[:, :, runs == 2, 5] *= 400.0
+    if kind == "wide400":
+        k[:, 2:5, :, 7] *= 2000.0
+    if kind in ("beyond", "all"):
+        k[:, :, runs == 3, 9] = 6e4 if dtype == torch.float16 else 1e15
+    if kind == "beyond":
+        k[:, 3:, :, 9] = 6e4 if dtype == torch.float16 else 1e15
+    if kind in ("query", "all"):
+        q[:, :3, :, 3] *= 3000.0
+    q, k = q.to(dtype), k.to(dtype).to(DEV)
+    for mode in ("snapkv", "rawsum"):
+        want = ops.snapkv_scores(q.repeat_interleave(3, dim=1).to(DEV), k, W, 0.1, 1, "maxpool", mode=mode)
+        got = ops.snapkv_scores(q.repeat_interleave(Hq // Hk, dim=1).to(DEV), k, W, 0.1, 1, "maxpool", mode=mode)
+        assert torch.equal(got.view(torch.int32), want.view(torch.int32)), mode
 
 
 @pytest.mark.parametrize("W,S,pool,pooling", [(64, 8270, 7, "avgpool"), (64, 8270, 7, "maxpool"), (64, 8232, 1, "maxpool"),
