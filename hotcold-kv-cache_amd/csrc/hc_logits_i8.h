@@ -197,8 +197,8 @@ __global__ __launch_bounds__(256) void qdigit_kernel(const T* __restrict__ q, co
     const float up = 1.f + 0x1p-14f, tiny = 1e-17f;
     QDigitRow o;
     o.scale = use ? ldexp(1.0, -sh) : 1.0;
-    o.norm = hi == 0 || use ? sqrtf(ss) * up + tiny : INFINITY;
-    o.resid = res * up + 2e-36f;
+    o.norm = hi == 0 ? 0.f : use ? sqrtf(ss) * up + tiny : INFINITY;     // (0: every product is 0)
+    o.resid = hi == 0 ? 0.f : res * up + 2e-36f;
     qrow[row + w] = o;
   }
   __syncthreads();
@@ -251,6 +251,7 @@ struct KDigits {
   i32x4 low[NS];   // the fifth digit, of weight 2^-8
   int f;           // scale 2^(f - kShift)
   int held;        // digits that hold every element exactly: 4, 5, or 0 if no five do
+  uint32_t zero;   // bit r: row r is all zero
   float norm;
 
   __device__ __forceinline__ void scan(const uint32_t (&w)[NP][4]) {
@@ -264,6 +265,9 @@ struct KDigits {
         mx = __builtin_elementwise_max(mx, __builtin_bit_cast(u16x2, w[p][i] & 0x7fff7fffu));
         ss = F::dot2(w[p][i], ss);
       }
+    uint64_t z = __ballot(__builtin_bit_cast(uint32_t, mx) == 0);     // the row's four lanes
+    z &= z >> 32;
+    zero = (uint32_t)(z & z >> 16) & 0xffffu;
     const uint32_t hi = reduce_cols(reduce_rows(__builtin_bit_cast(uint32_t, mx), MaxU16x2{}), MaxU16x2{});
     const int mb = __builtin_amdgcn_readfirstlane((int)max(hi & 0xffffu, hi >> 16));
     // a mantissa at 2 - 2^-7 or above would pass kFixMax
@@ -488,7 +492,7 @@ __global__ __launch_bounds__(256, 3) void logits_i8_kernel(
       const QDigitRow r = qrow[bh * wpad + w0 + tid];
       ssc[tid] = r.scale * lscale;
       sdel[tid] = ((double)r.norm * 0x1p-53 + (double)r.resid) * fabs(lscale) * 1.001;
-      float open = r.norm < INFINITY ? r.resid / r.norm : INFINITY;
+      float open = r.norm < INFINITY ? (r.norm > 0.f ? r.resid / r.norm : 0.f) : INFINITY;
 #pragma unroll
       for (int o = ROWS / 2; o > 0; o >>= 1) open += __shfl_xor(open, o, 64);
       if (tid == 0) open_s = open > NRB * kOpenRatio;
@@ -552,6 +556,7 @@ __global__ __launch_bounds__(256, 3) void logits_i8_kernel(
     const double del = dl * (double)kd.norm;
     const double sc = rs * __hiloint2double((1023 + kd.f - KFix<T>::kShift) << 20, 0);
     const int key = key0 + 4 * kk;
+    const uint32_t zero = kd.zero >> 4 * kk;
     float L[4];
     bool open = false;       // a logit that delta does not settle
 #pragma unroll
@@ -566,6 +571,10 @@ __global__ __launch_bounds__(256, 3) void logits_i8_kernel(
       L[i] = (float)__builtin_fma(d, sc, del);
       bool bad = !(lo == L[i]);
       if constexpr (!PLAIN) {
+        if (zero >> i & 1) {
+          L[i] = 0.f;
+          bad = false;
+        }
         if constexpr (MODE == HC_SCORE_SNAPKV)
           if (key + i > qpos0 + w) {
             L[i] = -INFINITY;
@@ -654,7 +663,7 @@ __global__ __launch_bounds__(256, 3) void logits_i8_kernel(
       kd.template digits<false>(raw);
       load(key0 + CHUNK);
       in = c + 1;
-      const bool plain = key0 + 16 <= S && (MODE != HC_SCORE_SNAPKV || key0 + 16 - 1 <= qpos0);
+      const bool plain = key0 + 16 <= S && (MODE != HC_SCORE_SNAPKV || key0 + 16 - 1 <= qpos0) && kd.zero == 0;
       // compiled apart, so that the common form is straight-line code
       redo_tiles(plain ? row_blocks(kd, key0, std::true_type{}, std::false_type{})
                        : row_blocks(kd, key0, std::false_type{}, std::false_type{}), key0);

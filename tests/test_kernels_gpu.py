@@ -591,9 +591,11 @@ def _digit_inputs(kind, shape_q, shape_k, dtype):
     g = torch.Generator().manual_seed(83)
     if kind == "outliers":
         k[..., :3] *= 40.0
-    elif kind == "mixed":         # runs of keys for four digits, five, and none at all
+    elif kind == "mixed":         # runs of keys for four digits, five, none at all, and zeros among each
         runs = torch.tensor([1.0, 300.0, 1e4, 1e9]).repeat_interleave(50)
         k[..., 1] = (k[..., 1] * runs.repeat(k.shape[2] // 200 + 1)[:k.shape[2]]).clamp(-6e4, 6e4)
+        k[:, :, ::37] = 0.0
+        k[:, :, 90:140] = 0.0
     elif kind == "wide":
         q, k = (t * torch.exp2(torch.randint(-12, 13, t.shape, generator=g).float()) for t in (q, k))
     elif kind == "tiny":
@@ -657,7 +659,7 @@ def test_long_window_scores_bit_exact(W, S, dtype, pool):
     assert torch.equal(got.nan_to_num(), want.nan_to_num())
 
 
-@pytest.mark.parametrize("kind", ["query", "wide400", "beyond", "all"])
+@pytest.mark.parametrize("kind", ["zero", "query", "wide400", "beyond", "all"])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("W,D,Hq", [(16, 64, 8), (32, 128, 8), (64, 128, 16), (50, 64, 8)])
 def test_window_logits_of_every_digit_form_over_many_chunks(kind, dtype, W, D, Hq):
@@ -668,6 +670,10 @@ def test_window_logits_of_every_digit_form_over_many_chunks(kind, dtype, W, D, H
     B, Hk, S = 6, 8, 64 * 250 + 13 if Hq == 8 else 64 * 120 + 13
     q, k = _randn((B, Hk, S, D), 95, torch.float32), _randn((B, Hk, S, D), 96, torch.float32)
     runs = torch.arange(S) // 48 % 5
+    if kind in ("zero", "all"):
+        k[:, :, runs == 1] = 0.0
+        k[:, :, ::91] = 0.0
+        q[:, 1, S - W // 2] = 0.0
     if kind in ("wide400", "all"):
         k[:, :, runs == 2, 5] *= 400.0
     if kind == "wide400":
