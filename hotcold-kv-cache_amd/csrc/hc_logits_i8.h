@@ -26,23 +26,22 @@
 // int8's, so 16 products cost a quarter of the one fp64 product.  Kernel times
 // (fp64 form -> this one, 8 KV heads of 128): window 64, 32k keys x 16 rows
 // f16 1243 -> 685 us, 64k x 4 bf16 with outlier channels 650 -> 400; window
-// 32, 32 layers of 8k keys 343 -> 207, one layer 21.6 -> 19.5 (bound by
+// 32, 32 layers of 8k keys 343 -> 207, one layer 20.8 -> 16.5 (bound by
 // latency); 32 heads of 5003 x 5003 (H2O) 1977 -> 1100.  What bounds it:
 // vector issue (per 16 keys x 64 rows about 270 instructions make the key
 // digits and 350 the logits, beside 128 matrix instructions of 16 cycles that
 // hide two vector instructions each) and the logits' stores, which are 14% of
 // the 32k launch and 27% of the H2O one.  Measured no faster: two key tiles
-// per wave, four waves per SIMD (spills), a row block's products interleaved
-// with the logits of the one before, and the keys' digits made once for all
-// row blocks.
+// per wave, a row block's products interleaved with the logits of the one
+// before, and the keys' digits made once for all row blocks.
 //
-// Off the common path (f16, 8 KV heads, the whole score call, against the fp64
-// form; 32k keys x 4 rows, window 64 | 8k x 32, window 32): four channels 100
-// times wider 411 -> 338 us | -, 400 times 412 -> 377 | 459 -> 447; a query
-// channel 100 times wider 409 -> 407 | 450 -> 390, 1000 times 409 -> 457 | 451 ->
-// 426; exponents over 24 binades 415 -> 460 | 453 -> 430.  So where all tiles are
-// the chain's it is from 6% faster to 12% slower than the fp64 kernel, whose
-// loop it is without that kernel's LDS for the whole window.
+// Off the common path (f16, 8 KV heads, the whole score call, fp64 form -> this
+// one; 32k keys x 4 rows, window 64 | 8k x 32, window 32): four channels 100
+// times wider 411 -> 343 us, 400 times 412 -> 384 | 459 -> 446; a query channel
+// 100 times wider 409 -> 415 | 450 -> 399, 1000 times 409 -> 463 | 451 -> 430;
+// exponents over 24 binades 415 -> 461 | 453 -> 432; logits that cancel exactly
+// 409 -> 495.  So where all tiles are the chain's it is from 5% faster to 13%
+// slower than the fp64 kernel: the same products, from a smaller LDS block.
 #pragma once
 #include <type_traits>
 
@@ -434,9 +433,10 @@ __device__ __forceinline__ void chain_tiles(const uint32_t (&w)[D / 32][4], F&& 
 // their own, the chain's with the queries in LDS for the whole workgroup: each
 // form keeps its registers, and the chain's tiles their matrix rate (the same
 // tiles redone one by one in place, the queries read from memory, took five
-// times the fp64 kernel).
+// times the fp64 kernel).  Up to 32 rows four waves fit a SIMD, and one 8k
+// layer's 1024 workgroups the chip at once (19.3 us with three).
 template <typename T, int MODE, int D, int NRB>
-__global__ __launch_bounds__(256, 3) void logits_i8_kernel(
+__global__ __launch_bounds__(256, MODE == HC_SCORE_SNAPKV && NRB < 4 ? 4 : 3) void logits_i8_kernel(
     const T* __restrict__ k, const T* const* __restrict__ k_rows, int64_t k_sb, int64_t k_sh, int64_t k_ss,
     uint32_t k_bytes, const double* __restrict__ qf, const int8_t* __restrict__ qd,
     const QDigitRow* __restrict__ qrow, int Hk, int S, int W, int wpad, double scaling, int cpw, int ld,
@@ -522,7 +522,8 @@ __global__ __launch_bounds__(256, 3) void logits_i8_kernel(
 
   // The products of row block nb against the chunk's keys; with LOW the fifth
   // digits' too, rest of weight 2^-8.
-  auto multiply = [&](const KDigits<T, D>& kd, i32x4 (&acc)[2 * kDigits - 1], i32x4& rest, int nb, auto low_c) {
+  auto multiply = [&](const KDigits<T, D>& kd, i32x4 (&acc)[2 * kDigits - 1], i32x4& rest, int lane, int nb,
+                      auto low_c) {
 #pragma unroll
     for (int j = 0; j < kDigits; ++j) {
       i32x4 q[NS];
@@ -548,7 +549,8 @@ __global__ __launch_bounds__(256, 3) void logits_i8_kernel(
   // before a key's position, no key past the last or all zero (its logits are
   // 0: with a delta of more they would all be redone).
   auto finish = [&](const KDigits<T, D>& kd, const i32x4 (&acc)[2 * kDigits - 1], const i32x4& rest, int key0,
-                    uint32_t& redo, int nb, auto plain_c, auto low_c) {
+                    uint32_t& redo, int lane, int nb, auto plain_c, auto low_c) {
+    const int col = lane & 15, kk = lane >> 4;
     constexpr bool PLAIN = decltype(plain_c)::value, LOW = decltype(low_c)::value;
     const int w = 16 * nb + col;
     const double rs = ssc[w], dl = sdel[w];
@@ -605,13 +607,13 @@ __global__ __launch_bounds__(256, 3) void logits_i8_kernel(
       }
     }
   };
-  auto row_blocks = [&](const KDigits<T, D>& kd, int key0, auto plain_c, auto low_c) {
+  auto row_blocks = [&](const KDigits<T, D>& kd, int key0, int lane, auto plain_c, auto low_c) {
     uint32_t redo = 0;
 #pragma unroll
     for (int nb = 0; nb < NRB; ++nb) {
       i32x4 acc[2 * kDigits - 1], rest;
-      multiply(kd, acc, rest, nb, low_c);
-      finish(kd, acc, rest, key0, redo, nb, plain_c, low_c);
+      multiply(kd, acc, rest, lane, nb, low_c);
+      finish(kd, acc, rest, key0, redo, lane, nb, plain_c, low_c);
       // side by side, two row blocks with a fifth digit would need more
       // registers than the common form
       if constexpr (decltype(low_c)::value) __builtin_amdgcn_sched_barrier(0);
@@ -640,10 +642,10 @@ __global__ __launch_bounds__(256, 3) void logits_i8_kernel(
   // Chunks whose keys need a fifth digit, and those that only the fp64 chain
   // does, are left for the loops below (bit c of wide and hard).  After two at
   // the start the rest is left unseen: where all are, looking costs a read of
-  // the keys.  `in` is the chunk that raw holds.
+  // the keys.
   const uint32_t all = (1u << nmul) - 1;
   uint32_t wide = 0, hard = open_rows ? all : 0;
-  int in = 0;
+  int nopen = 0;
   if (!open_rows)
     for (int c = 0; c < nmul; ++c) {
       // the row blocks' LDS reads repeat for every chunk: hoisted, they would
@@ -653,35 +655,42 @@ __global__ __launch_bounds__(256, 3) void logits_i8_kernel(
       kd.scan(raw);
       if (kd.held != kDigits) {    // wave-uniform
         wide |= 1u << c;
-        if (wide == 3) wide = all;
-        in = c;
-        if (c + 1 == nmul || wide == all) break;
+        if (wide == 3) {
+          wide = all;
+          break;
+        }
         load(key0 + CHUNK);
         key0 += CHUNK;
         continue;
       }
       kd.template digits<false>(raw);
       load(key0 + CHUNK);
-      in = c + 1;
       const bool plain = key0 + 16 <= S && (MODE != HC_SCORE_SNAPKV || key0 + 16 - 1 <= qpos0) && kd.zero == 0;
       // compiled apart, so that the common form is straight-line code
-      redo_tiles(plain ? row_blocks(kd, key0, std::true_type{}, std::false_type{})
-                       : row_blocks(kd, key0, std::false_type{}, std::false_type{}), key0);
+      const uint32_t redo = plain ? row_blocks(kd, key0, lane, std::true_type{}, std::false_type{})
+                                  : row_blocks(kd, key0, lane, std::false_type{}, std::false_type{});
+      redo_tiles(redo, key0);
       key0 += CHUNK;
+      // nothing settled in two chunks (logits that cancel to a few bits): the
+      // rest goes to the chain
+      nopen = redo == (1u << (nw + 15) / 16) - 1 ? nopen + 1 : 0;
+      if (nopen == 2) {
+        hard |= all & ~((2u << c) - 1);
+        break;
+      }
     }
-  // last first: it may be in
   for (uint32_t left = wide; left;) {
     __asm__ volatile("" ::: "memory");
-    const int c = 31 - __clz(left), at = chunk(c);
-    left &= ~(1u << c);
-    // (not loaded ahead: the fifth digit takes the registers)
-    if (in != c) load(at);
-    in = c;
+    const int c = __ffs(left) - 1, at = chunk(c);
+    left &= left - 1;
+    load(at);                    // (not ahead: the fifth digit takes the registers)
     KDigits<T, D> kd;
     kd.scan(raw);
     if (kd.held) {               // wave-uniform
       kd.template digits<true>(raw);
-      redo_tiles(row_blocks(kd, at, std::false_type{}, std::true_type{}), at);
+      int l = lane;              // (as in chain_tiles: nothing hoisted)
+      __asm__ volatile("" : "+v"(l));
+      redo_tiles(row_blocks(kd, at, l, std::false_type{}, std::true_type{}), at);
       continue;
     }
     hard |= 1u << c;
@@ -707,8 +716,7 @@ __global__ __launch_bounds__(256, 3) void logits_i8_kernel(
       for (int t = 0; t < PB; ++t)
 #pragma unroll
         for (int i = 0; i < 4; ++i) top[t][i] = -INFINITY;
-      if (left && __ffs(left) - 1 != in) load(chunk(__ffs(left) - 1));
-      in = -1;
+      if (left) load(chunk(__ffs(left) - 1));
       while (left) {             // wave-uniform
         const int at = chunk(__ffs(left) - 1);
         left &= left - 1;

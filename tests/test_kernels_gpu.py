@@ -659,7 +659,7 @@ def test_long_window_scores_bit_exact(W, S, dtype, pool):
     assert torch.equal(got.nan_to_num(), want.nan_to_num())
 
 
-@pytest.mark.parametrize("kind", ["zero", "query", "wide400", "beyond", "all"])
+@pytest.mark.parametrize("kind", ["zero", "query", "wide400", "beyond", "cancel", "all"])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("W,D,Hq", [(16, 64, 8), (32, 128, 8), (64, 128, 16), (50, 64, 8)])
 def test_window_logits_of_every_digit_form_over_many_chunks(kind, dtype, W, D, Hq):
@@ -684,7 +684,12 @@ def test_window_logits_of_every_digit_form_over_many_chunks(kind, dtype, W, D, H
         k[:, 3:, :, 9] = 6e4 if dtype == torch.float16 else 1e15
     if kind in ("query", "all"):
         q[:, :3, :, 3] *= 3000.0
-    q, k = q.to(dtype), k.to(dtype).to(DEV)
+    q, k = q.to(dtype), k.to(dtype)
+    if kind == "cancel":
+        q[..., D // 2:] = q[..., :D // 2]
+        k[:, :4, :, D // 2:] = -k[:, :4, :, :D // 2]
+        k[:, 4:, 300:3000, D // 2:] = -k[:, 4:, 300:3000, :D // 2]
+    k = k.to(DEV)
     for mode in ("snapkv", "rawsum"):
         want = ops.snapkv_scores(q.repeat_interleave(3, dim=1).to(DEV), k, W, 0.1, 1, "maxpool", mode=mode)
         got = ops.snapkv_scores(q.repeat_interleave(Hq // Hk, dim=1).to(DEV), k, W, 0.1, 1, "maxpool", mode=mode)
