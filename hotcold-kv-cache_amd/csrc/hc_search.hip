@@ -583,7 +583,11 @@ __global__ __launch_bounds__(kIdxThreads) void index_select_kernel(IndexSearchAr
 // select) and the candidates collected again, and if they are still too many
 // (many near-ties) the workgroup scores every slot exactly and runs the exact
 // selection.  The candidates' exact fp64 scores, ranked by (score descending,
-// logical index ascending), give the exact hits.
+// logical index ascending), give the exact hits.  Keys with a large shared mean
+// crowd a few bins: 20 times the spread of each 29.3 us where separate keys take
+// 21.3 (15360 tokens); with every key equal the histogram's atomics go one by
+// one, 9 of the 199 us that the exact selection takes (counting a wave's equal
+// bins together saves those and costs every other search 1 to 2 us).
 //
 // One workgroup's chain of dependent steps bounds it (8 searches of 64 in
 // 15360 tokens, a CU each): the keys are read once into registers, the query
@@ -594,6 +598,11 @@ constexpr int kBins = 2048;      // of 2^-10 in the score, from -1
 constexpr uint32_t kBinBase = 1u << 29;
 constexpr int kBinShift = 19;
 constexpr int kScoreLanes = 8;   // lanes per candidate
+// Up to this many candidates are scored by eight lanes each and ranked by count;
+// more by a thread each and sorted (8 searches of 64 in 1000 tokens, us: 256
+// candidates 23.0 against 26.2, 400 candidates 40.0 against 28.5, 1000 125
+// against 38).
+constexpr int kRankMax = 256;
 
 // Sum of the products q_d x_d over the dimensions in order, in fp64 (products
 // of two floats are exact): lane j of a candidate's eight holds dimensions
@@ -687,7 +696,13 @@ __global__ __launch_bounds__(kIdxThreads) void index_select16_kernel(IndexSearch
 #pragma unroll
     for (int w = 0; w < kIdxThreads / 64; ++w) incl += w < wave ? wave_tot[w] : 0u;
     const uint32_t excl = incl - v, want = (uint32_t)m;
-    if (excl < want && incl >= want) bin_s = excl + c0 >= want ? kBins - 1 - 2 * tid : kBins - 2 - 2 * tid;
+    if (excl < want && incl >= want) {
+      const bool upper = excl + c0 >= want;
+      bin_s = kBins - (upper ? 1 : 2) - 2 * tid;
+      // more than fit in the m-th score's bin and above: not collected from it
+      const uint32_t n = upper ? excl + c0 : incl;
+      if (n > kCandX) y.n_c = (int)n;
+    }
     __syncthreads();
   }
   // the smallest key whose slot can score the low end of key `low` minus
@@ -701,9 +716,12 @@ __global__ __launch_bounds__(kIdxThreads) void index_select16_kernel(IndexSearch
     const int i = append_slot(&y.n_c, want);
     if (i >= 0 && i < kCandX) y.cp[i] = p;
   };
-  const uint32_t from = first_key(bin_s ? kBinBase + ((uint32_t)bin_s << kBinShift) : 0u);
-  every([&](int p, uint32_t k, bool in) __attribute__((always_inline)) { add(p, in && k >= from); });
-  __syncthreads();
+  if (y.n_c == 0) {     // uniform
+    const uint32_t from = first_key(bin_s ? kBinBase + ((uint32_t)bin_s << kBinShift) : 0u);
+    __syncthreads();
+    every([&](int p, uint32_t k, bool in) __attribute__((always_inline)) { add(p, in && k >= from); });
+    __syncthreads();
+  }
   if (y.n_c > kCandX) {  // uniform
     int remaining;
     const uint32_t T = radix_select<uint32_t>(kb32, size, m, tid, y.ck, kCand, y.rs, remaining);
@@ -721,7 +739,7 @@ __global__ __launch_bounds__(kIdxThreads) void index_select16_kernel(IndexSearch
     select_exact(a, b, vh, kb, m, tid, sm.x);
     return;
   }
-  if (a.VD == 128 || a.VD == 64 || a.VD == 32) {   // uniform
+  if (nc <= kRankMax && (a.VD == 128 || a.VD == 64 || a.VD == 32)) {   // uniform
     for (int i0 = 0; i0 < nc; i0 += kIdxThreads / kScoreLanes) {
       const int i = i0 + tid / kScoreLanes, p = y.cp[min(i, nc - 1)];
       const double sc = a.VD == 128 ? exact_score_lanes<4>(vb, qv, p, 128)
@@ -738,6 +756,18 @@ __global__ __launch_bounds__(kIdxThreads) void index_select16_kernel(IndexSearch
       y.ckey[i] = ordered_key(exact_score(vb, qv, p, a.VD));
       y.cl[i] = logical(p);
     }
+  }
+  if (nc > kRankMax) {    // uniform
+    int P = 1;
+    while (P < nc) P <<= 1;
+    for (int i = nc + tid; i < P; i += kIdxThreads) {
+      y.ckey[i] = 0;
+      y.cl[i] = 0x7fffffff;
+    }
+    __syncthreads();
+    sort_ranked<kCandX>(y.ckey, y.cl, P, tid);
+    write_hits(a, b, vh, m, y.cl, tid);
+    return;
   }
   __syncthreads();
   // Rank by count: `per` neighbouring lanes share a candidate's comparisons.

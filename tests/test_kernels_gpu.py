@@ -1526,6 +1526,31 @@ def test_device_index_fp16_pass_sizes(D, tokens, R):
         assert (hits[0][..., min(R, tokens):] == -1).all() and (hits[0][..., :min(R, tokens)] >= 0).all()
 
 
+@pytest.mark.parametrize("n", [1, 240, 300, 1100, 2040, 2060, 6000])
+@pytest.mark.parametrize("D", [128, 96])
+def test_device_index_fp16_pass_crowded(n, D):
+    """n of 6000 vectors within two bins and 2 delta of each other (the first
+    third of them equal): ranked by count, sorted, and more than are re-scored
+    at once; the hits are the exact scan's, older slots first among equals."""
+    from hotcold_kv.device_index import DeviceIndex
+    g = torch.Generator().manual_seed(n)
+    k, q = torch.randn((1, 2, 6000, D), generator=g), torch.randn((1, 2, D), generator=g)
+    u = q / q.norm(dim=-1, keepdim=True)
+    w = torch.randn((1, 2, n, D), generator=g)
+    w = w - (w * u[:, :, None]).sum(-1, keepdim=True) * u[:, :, None]
+    c = 0.9 + 0.0005 * torch.rand((1, 2, n, 1), generator=g)
+    near = c * u[:, :, None] + (1 - c * c).sqrt() * w / w.norm(dim=-1, keepdim=True)
+    near[:, :, : n // 3] = near[:, :, :1]
+    k[:, :, torch.randperm(6000, generator=g)[:n]] = near
+    dix = DeviceIndex(1, 2, D, D, 2, 6000, DEV)
+    dix.add(k.to(DEV), np.arange(6000, dtype=np.int64)[None])
+    for R in (1, 64, 500):
+        hits = [torch.empty((1, 2, R), dtype=torch.int64, device=DEV) for _ in range(2)]
+        dix.search(q.to(DEV), R, hits[0])
+        dix.search(q.to(DEV), R, hits[1], pass16=False)
+        assert torch.equal(hits[0], hits[1]), R
+
+
 @pytest.mark.parametrize("per_head,faiss_dim,normalize", [(False, 32, True), (True, 64, True), (True, 96, True),
                                                          (True, 64, False)])
 def test_scheduled_device_search_equals_the_host_search(per_head, faiss_dim, normalize):
