@@ -40,8 +40,9 @@
 // times wider 411 -> 343 us, 400 times 412 -> 384 | 459 -> 446; a query channel
 // 100 times wider 409 -> 415 | 450 -> 399, 1000 times 409 -> 463 | 451 -> 430;
 // exponents over 24 binades 415 -> 461 | 453 -> 432; logits that cancel exactly
-// 409 -> 495.  So where all tiles are the chain's it is from 5% faster to 13%
-// slower than the fp64 kernel: the same products, from a smaller LDS block.
+// 409 -> 577.  So where all tiles are known to be the chain's it is from 5% faster
+// to 13% slower than the fp64 kernel (the same products, from a smaller LDS
+// block); where only the digits show it, they come on top.
 #pragma once
 #include <type_traits>
 
@@ -118,27 +119,28 @@ struct SumF32 {
 
 // The group-mean queries with their digits, and qmean_kernel's resets of the
 // row maxima, the NaN flag and the padding statistics (zero rows past W).
-// grid (wpad / 4, Hk, B), block 256, one wave per row; lane l owns dims
+// grid (wpad / RB, Hk, B), block 64 RB, one wave per row; lane l owns dims
 // E l .. E l + E - 1.  Both leave in the order that the matrix instructions read
-// them, 16 rows to a block, through LDS so that four rows' 16-byte pieces go out
+// them, 16 rows to a block, through LDS so that RB rows' 16-byte pieces go out
 // together:
 //   qf [row block][dims 8u .. 8u + 7][lane][2], lane (kk, row) holding dims
 //      8u + kk and 8u + 4 + kk: two k-steps of the fp64 chain;
 //   qd [row block][digit][k-step of 64][lane][16], lane (kk, row) holding dims
 //      8 * (kk + 4 * t) + r of the pieces t = 2s, 2s + 1 of k-step s.
-// Bound by its stores (12 bytes per element).
-template <typename T, int D>
-__global__ __launch_bounds__(256) void qdigit_kernel(const T* __restrict__ q, const T* const* __restrict__ q_rows,
+// Bound by its stores (12 bytes per element): 87 us for 32 heads of 5003 rows at
+// RB = 16, 4.2 for 8 heads of 32 at RB = 4.
+template <typename T, int D, int RB>
+__global__ __launch_bounds__(64 * RB) void qdigit_kernel(const T* __restrict__ q, const T* const* __restrict__ q_rows,
                                                      int64_t q_sb, int64_t q_sh, int64_t q_ss, int64_t q_row0, int Hq,
                                                      int Hk, int W, int wpad, double* __restrict__ qf,
                                                      uint32_t* __restrict__ rmax, RowStat* __restrict__ rstat,
                                                      uint32_t* __restrict__ nan_flag, int8_t* __restrict__ qd,
                                                      QDigitRow* __restrict__ qrow) {
   constexpr int E = D / 64;
-  __shared__ double sx[4][D + 4];
-  __shared__ i32x4 sd[D * kDigits / 4];
+  __shared__ double sx[RB][D + 4];
+  __shared__ i32x4 sd[RB * D * kDigits / 16];
   const int tid = threadIdx.x, lane = tid & 63, r = tid >> 6;
-  const int w = (int)blockIdx.x * 4 + r, h = blockIdx.y, b = blockIdx.z;
+  const int w = (int)blockIdx.x * RB + r, h = blockIdx.y, b = blockIdx.z;
   const int64_t bh = (int64_t)b * Hk + h, row = bh * wpad;
   const int wst = (int)cdiv(W, kStatPad) * kStatPad;
   if (lane == 0 && w == 0) nan_flag[bh] = 0;
@@ -183,12 +185,13 @@ __global__ __launch_bounds__(256) void qdigit_kernel(const T* __restrict__ q, co
     u[e] = ((uint32_t)v + kBalance) ^ kBalance;
   }
   const int d = lane * E, t = d >> 5;
-  // sd: [digit][k-step][kk][row of 4][16]
-  int8_t* dst = reinterpret_cast<int8_t*>(sd) + (t >> 1) * 256 + (((d >> 3) & 3) * 4 + r) * 16 + (t & 1) * 8 + (d & 7);
+  // sd: [digit][k-step][kk][row of RB][16]
+  int8_t* dst = reinterpret_cast<int8_t*>(sd) + ((t >> 1) * 4 + ((d >> 3) & 3)) * RB * 16 + r * 16 + (t & 1) * 8 +
+                (d & 7);
 #pragma unroll
   for (int j = 0; j < kDigits; ++j)
 #pragma unroll
-    for (int e = 0; e < E; ++e) dst[j * (D / 64) * 256 + e] = (int8_t)(u[e] >> (8 * j));
+    for (int e = 0; e < E; ++e) dst[j * (D / 64) * RB * 64 + e] = (int8_t)(u[e] >> (8 * j));
   ss = __uint_as_float(reduce_cols(reduce_rows(__float_as_uint(ss), SumF32{}), SumF32{}));
   res = __uint_as_float(reduce_cols(reduce_rows(__float_as_uint(res), SumF32{}), SumF32{}));
   if (lane == 0) {
@@ -202,15 +205,15 @@ __global__ __launch_bounds__(256) void qdigit_kernel(const T* __restrict__ q, co
   }
   __syncthreads();
   const int64_t at = (row + (w >> 4) * 16) * D;      // the row block
-  const int r0 = (int)blockIdx.x % 4 * 4;
+  const int r0 = (int)blockIdx.x * RB % 16;
   doublex2* of = reinterpret_cast<doublex2*>(qf + at);
   i32x4* od = reinterpret_cast<i32x4*>(qd + at * kDigits);
 #pragma unroll
-  for (int i = tid; i < 2 * D; i += 256) {           // piece i: dims 8 (i / 16) + (i / 4) % 4, row i % 4
-    const int c = (i >> 4) * 8 + ((i >> 2) & 3);
-    of[(i >> 2) * 16 + r0 + (i & 3)] = doublex2{sx[i & 3][c], sx[i & 3][c + 4]};
+  for (int i = tid; i < RB * D / 2; i += 64 * RB) {  // piece i: dims 8 (i / 4 RB) + (i / RB) % 4, row i % RB
+    const int c = i / (4 * RB) * 8 + i / RB % 4;
+    of[i / RB * 16 + r0 + i % RB] = doublex2{sx[i % RB][c], sx[i % RB][c + 4]};
   }
-  if (tid < D * kDigits / 4) od[(tid >> 2) * 16 + r0 + (tid & 3)] = sd[tid];
+  if (tid < RB * D * kDigits / 16) od[tid / RB * 16 + r0 + tid % RB] = sd[tid];
 }
 
 // Fixed point of key rows: |x| * 2^(kShift - f) <= kFixMax for every element,
@@ -445,8 +448,7 @@ __global__ __launch_bounds__(256, MODE == HC_SCORE_SNAPKV && NRB < 4 ? 4 : 3) vo
   constexpr int PB = NRB < 2 ? NRB : 2;       // row blocks per pass over the hard chunks
   constexpr int SQ_DIGITS = NRB * kDigits * NS * 64, SQ_CHAIN = PB * 8 * D;
   __shared__ i32x4 sq[SQ_DIGITS > SQ_CHAIN ? SQ_DIGITS : SQ_CHAIN];
-  __shared__ double ssc[ROWS];       // row scale times the logit scale
-  __shared__ double sdel[ROWS];      // a key of 2-norm 1's delta against the row
+  __shared__ doublex2 srow[ROWS];    // row scale times the logit scale; a key of 2-norm 1's delta against the row
   __shared__ uint32_t redk[ROWS];
   __shared__ int open_s;             // the rows' residuals leave most tiles open
   __shared__ int hard_s;             // a wave has hard chunks
@@ -490,8 +492,7 @@ __global__ __launch_bounds__(256, MODE == HC_SCORE_SNAPKV && NRB < 4 ? 4 : 3) vo
     const double lscale = MODE == HC_SCORE_SNAPKV ? scaling : 1.0 / scaling;
     if (tid < ROWS) {
       const QDigitRow r = qrow[bh * wpad + w0 + tid];
-      ssc[tid] = r.scale * lscale;
-      sdel[tid] = ((double)r.norm * 0x1p-53 + (double)r.resid) * fabs(lscale) * 1.001;
+      srow[tid] = doublex2{r.scale * lscale, ((double)r.norm * 0x1p-53 + (double)r.resid) * fabs(lscale) * 1.001};
       float open = r.norm < INFINITY ? (r.norm > 0.f ? r.resid / r.norm : 0.f) : INFINITY;
 #pragma unroll
       for (int o = ROWS / 2; o > 0; o >>= 1) open += __shfl_xor(open, o, 64);
@@ -553,7 +554,8 @@ __global__ __launch_bounds__(256, MODE == HC_SCORE_SNAPKV && NRB < 4 ? 4 : 3) vo
     const int col = lane & 15, kk = lane >> 4;
     constexpr bool PLAIN = decltype(plain_c)::value, LOW = decltype(low_c)::value;
     const int w = 16 * nb + col;
-    const double rs = ssc[w], dl = sdel[w];
+    const doublex2 row = srow[w];
+    const double rs = row[0], dl = row[1];
     const uint64_t live = ((1ull << min(max(nw - 16 * nb, 0), 16)) - 1) * 0x0001000100010001ull;   // real rows' lanes
     const double del = dl * (double)kd.norm;
     const double sc = rs * __hiloint2double((1023 + kd.f - KFix<T>::kShift) << 20, 0);
@@ -645,7 +647,6 @@ __global__ __launch_bounds__(256, MODE == HC_SCORE_SNAPKV && NRB < 4 ? 4 : 3) vo
   // the keys.
   const uint32_t all = (1u << nmul) - 1;
   uint32_t wide = 0, hard = open_rows ? all : 0;
-  int nopen = 0;
   if (!open_rows)
     for (int c = 0; c < nmul; ++c) {
       // the row blocks' LDS reads repeat for every chunk: hoisted, they would
@@ -669,15 +670,11 @@ __global__ __launch_bounds__(256, MODE == HC_SCORE_SNAPKV && NRB < 4 ? 4 : 3) vo
       // compiled apart, so that the common form is straight-line code
       const uint32_t redo = plain ? row_blocks(kd, key0, lane, std::true_type{}, std::false_type{})
                                   : row_blocks(kd, key0, lane, std::false_type{}, std::false_type{});
-      redo_tiles(redo, key0);
+      // (with every row block open, as where logits cancel to a few bits, the
+      // chain's loop does them faster)
+      if (NRB > 1 && redo == (1u << NRB) - 1) hard |= 1u << c;
+      else redo_tiles(redo, key0);
       key0 += CHUNK;
-      // nothing settled in two chunks (logits that cancel to a few bits): the
-      // rest goes to the chain
-      nopen = redo == (1u << (nw + 15) / 16) - 1 ? nopen + 1 : 0;
-      if (nopen == 2) {
-        hard |= all & ~((2u << c) - 1);
-        break;
-      }
     }
   for (uint32_t left = wide; left;) {
     __asm__ volatile("" ::: "memory");
