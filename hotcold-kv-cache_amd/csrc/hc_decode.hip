@@ -520,7 +520,6 @@ static int decode_impl(int dtype, int64_t B, int64_t Hq, int64_t Hk, int64_t D, 
   a.part = reinterpret_cast<float*>(ws + lay.part_off);
   a.scores = with_evict ? reinterpret_cast<float*>(ws + lay.scores_off) : nullptr;
   a.ml = with_evict ? reinterpret_cast<float*>(ws + lay.ml_off) : nullptr;
-  a.evict_min = evict_loss ? reinterpret_cast<unsigned long long*>(ws + lay.min_off) : nullptr;
   a.B = (int)B; a.Hq = (int)Hq; a.Hk = (int)Hk; a.G = G; a.S = (int)S;
   a.splits = splits;
   a.keys_per_split = (int)shape.kps;
@@ -536,7 +535,7 @@ static int decode_impl(int dtype, int64_t B, int64_t Hq, int64_t Hk, int64_t D, 
     a.pos_new = ap->pos_new; a.posn_sb = ap->posn_sb; a.pos_dst = ap->pos_dst; a.posd_sb = ap->posd_sb;
   } else {
     a.k_new = a.v_new = a.p_new = nullptr;
-    a.p_dst = nullptr;
+    a.evict_min = evict_loss ? reinterpret_cast<unsigned long long*>(ws + lay.min_off) : nullptr;
     a.pos_new = nullptr;
     a.pos_dst = nullptr;
   }

@@ -94,7 +94,12 @@ struct DecodeArgs {
   float* part;         // [units][splits][G*D + 2*G] split partials (splits > 1)
   float* scores;       // optional [B][Hq][S] log2-domain logits (eviction score)
   float* ml;           // optional [B][Hq][2] final (max, sum)
-  void* p_dst;         // fused append: the pre-RoPE key's and position's destinations
+  union {              // (the eviction score is not computed with a fused append)
+    void* p_dst;       // fused append: the pre-RoPE key's and position's destinations
+    // Eviction score: per batch row its running minimum and its count of
+    // finished workgroups (evict_score_kernel), reset by this launch.
+    unsigned long long* evict_min;
+  };
   int64_t pd_sb, pd_sh, pd_ss;
   int64_t* pos_dst;
   int64_t posd_sb;
@@ -105,10 +110,8 @@ struct DecodeArgs {
   // previous launch (epoch itself if not known).
   unsigned long long* counters;
   uint32_t epoch, prev_epoch;
-  // Eviction score: per batch row its running minimum and its count of
-  // finished workgroups (evict_score_kernel), reset by this launch.
-  unsigned long long* evict_min;
 };
+static_assert(sizeof(DecodeArgs) == 416, "every launch copies the block: its fields are what some launch reads");
 static_assert(offsetof(DecodeArgs, Hq) + sizeof(int) <= 128, "the first loads' fields must fit bytes 0-127");
 static_assert(offsetof(DecodeArgs, B) == 128 && offsetof(DecodeArgs, cur_pos) + sizeof(void*) <= 256,
               "the prologue's other fields must fit bytes 128-255");
