@@ -190,14 +190,8 @@ struct DetExp {
   // double, so the scaling is exact (v_ldexp_f64, one instruction; building
   // the factor from exponent bits measured slower).
   __device__ __forceinline__ static double scale(double p, uint32_t j) { return __builtin_ldexp(p, (int)j); }
-  // The contract's value: exp(x) for x >= -708, else +0.
-  __device__ __forceinline__ double operator()(double x) const {
-    uint32_t k;
-    const double p = poly<0>(x, k);
-    return x >= -708.0 ? scale(p, k) : 0.0;  // false for -inf and NaN
-  }
-  // The contract's value, except that arguments below -708 (-inf and NaN too)
-  // give exp(-708), about 3.3e-308, instead of 0.
+  // The contract's value (exp(x) for x >= -708, else +0), except that arguments
+  // below -708 (-inf and NaN too) give exp(-708), about 3.3e-308, instead of 0.
   __device__ __forceinline__ double floored(double x) const {
     uint32_t k;
     const double p = poly<0>(x, k);

@@ -171,7 +171,6 @@ __device__ __forceinline__ uint32_t fixed_key32(float s) {
   return x <= 0.0 ? 0u : (x >= 4294967295.0 ? 0xffffffffu : (uint32_t)x);
 }
 __device__ __forceinline__ double fixed_key_low(uint32_t k) { return (double)k / kFixScale - 2.0; }
-__device__ __forceinline__ double fixed_key_high(uint32_t k) { return ((double)k + 1.0) / kFixScale - 2.0; }
 
 // The norm of the VD values staged at qv (VD a multiple of 4): one fp64 chain
 // in dimension order, by one wave.  16 values are read before any is used: read
@@ -199,7 +198,8 @@ __device__ __forceinline__ void query_norm(const float* qv, int VD, int lane, do
 // The query of (row b, head vh), cropped or zero-padded to VD and (with
 // normalize_q) divided by its norm, as the stored vectors are: the raw values
 // are staged in LDS by all threads, the norm is one fp64 chain over them in
-// dimension order (thread 0), and each dimension is divided by its own thread.
+// dimension order (query_norm, by the first wave), and each dimension is divided
+// by its own thread.
 // Ends with a barrier.
 __device__ void stage_query(const IndexSearchArgs& a, int b, int vh, int tid, int nthreads, float* qv,
                             double* den_s) {

@@ -523,9 +523,15 @@ __global__ __launch_bounds__(256) void rowsum_kernel(const float* __restrict__ l
 // SGPRs, with no LDS staging and no per-row branch.
 constexpr int kImpRows = 8;
 // Windows from this many rows on take imp_split_kernel when there is no
-// pooling: with the window the prompt it is the faster from the smallest sizes
-// measured (32 heads of 401: 59 -> 18 us, 1001: 128 -> 51).  Observation
-// windows (8 to 64 rows) have keys enough for one thread each.
+// pooling, unless one thread per key fills the chip and the chains are of like
+// length: at least kPoolMinWaves waves of keys and a window of at most a quarter
+// of the prompt.  Observation windows (8 to 64 rows) have keys enough for one
+// thread each.  Importance kernel, split against one thread per key (us, 8 KV
+// heads; window 256 | 2048): 1 x 4096 keys 15, 35 | 93, 238; 1 x 16384 42, 44 |
+// 304, 329; 1 x 32768 66, 63 | 529, 506; 4 x 32768 268, 227 | 2184, 1882.  Half
+// the prompt, 4 x 16384: 3652, 3952; the prompt, 32 heads of 8192: 1363, 1912,
+// of 401: 18, 59.
+constexpr int64_t kPoolMinWaves = 4096;
 constexpr int kSplitMinW = 256;
 
 // One key's importance: the fma chain over rows [wbeg, W) of the logits
@@ -864,7 +870,8 @@ static void launch_score(const ScoreLayout& lay, char* ws, int mode, int64_t B, 
       hipLaunchKernelGGL(rowsum_kernel<false>, g, dim3(256), 0, st, (const float*)logits, (const uint32_t*)rmax,
                          (int)Hk, (int)S, (int)lay.ld, (int)W, nsplit, rstat, nan_flag);
   }
-  if (mode == HC_SCORE_SNAPKV && P == 0 && W >= kSplitMinW) {
+  const bool key_threads = cdiv(S, 64) * Hk * B >= kPoolMinWaves && W <= S / 4;
+  if (mode == HC_SCORE_SNAPKV && P == 0 && W >= kSplitMinW && !key_threads) {
     hipLaunchKernelGGL(imp_split_kernel, dim3((unsigned)cdiv(S, 64), (unsigned)Hk, (unsigned)B), dim3(256), 0, st,
                        (const float*)logits, (const RowStat*)rstat, (const uint32_t*)nan_flag, (int)Hk, (int)S,
                        (int)lay.ld, (int)W, scores);

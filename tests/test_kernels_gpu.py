@@ -564,10 +564,10 @@ SCORE_CASES = [
     (1, 4, 4, 20, 16, 32, torch.float32, 7, "maxpool"),      # window longer than the prompt
     # few rows: each row sum split across 4 waves, S not a multiple of 256
     (1, 8, 2, 3000, 64, 7, torch.float16, 7, "maxpool"),     # S % 4 == 0 (vector row loads)
-    (1, 8, 2, 3001, 128, 7, torch.bfloat16, 5, "avgpool"),   # S % 4 != 0 (scalar row loads)
+    (1, 8, 2, 3001, 128, 7, torch.bfloat16, 5, "avgpool"),   # S % 16 != 0: rows padded in the workspace
     # enough rows and keys for several 128-key chunks per logits workgroup
     (8, 32, 8, 4160, 128, 32, torch.float16, 7, "maxpool"),
-    # a long window without pooling: importance over mirrored key pairs
+    # a long window without pooling: the importance chains split over four waves
     (1, 4, 2, 2500, 64, 1100, torch.float16, 1, "maxpool"),
     (2, 2, 2, 1301, 32, 1301, torch.float32, 1, "maxpool"),
 ]
@@ -708,6 +708,41 @@ def test_early_row_without_finite_logit_makes_every_score_nan(W, S, pool, poolin
     assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.nan_to_num(), want.nan_to_num())
     if pooling == "avgpool":
         assert torch.isnan(got[:, 0]).all() and not torch.isnan(got[:, 1]).any()
+
+
+@pytest.mark.parametrize("W", [255, 256, 2076, 2077, 2100])
+def test_long_window_of_a_long_prompt_scores_alike_alone_and_batched(W):
+    """Four rows of 8305 keys fill the chip with one thread per key, and windows
+    up to a quarter of them take it; a row alone is split over waves."""
+    q, k = _randn((4, 8, 8305, 64), 99, torch.float16).to(DEV), _randn((4, 8, 8305, 64), 100, torch.float16).to(DEV)
+    q[2, 3, 8305 - W + 1] = float("nan")
+    got = ops.snapkv_scores(q, k, W, 0.125, 1, "maxpool")
+    for b in range(4):
+        want = ops.snapkv_scores(q[b:b + 1], k[b:b + 1], W, 0.125, 1, "maxpool")
+        assert torch.equal(got[b].isnan(), want[0].isnan()) and torch.equal(got[b].nan_to_num(), want[0].nan_to_num())
+    assert torch.isnan(got[2, 3]).all() and int(torch.isnan(got).sum()) == 8305
+
+
+@pytest.mark.parametrize("W,S,pool", [(23169, 23169, 1), (16384, 32767, 5)])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+def test_scores_of_unpadded_logits_rows(W, S, pool, dtype):
+    """Windows whose logits rows padded to 16 keys would pass 2 GiB a head keep
+    rows of S floats, aligned to one float only.  The digits' kernel against the
+    fp64 one (a group of three equal heads) bit for bit, and both against fp64
+    probabilities: a logit rounded to fp32 (|L| < 8) is off by 2^-22, a score by
+    that share of it, and the scores are rounded once more."""
+    assert W * S < 1 << 29 <= W * ((S + 15) // 16 * 16)
+    q, k = _randn((1, 1, S, 64), 97, dtype).to(DEV), _randn((1, 1, S, 64), 98, dtype).to(DEV)
+    got = ops.snapkv_scores(q, k, W, 0.125, pool, "avgpool")
+    assert torch.equal(got, ops.snapkv_scores(q.expand(1, 3, S, 64).contiguous(), k, W, 0.125, pool, "avgpool"))
+    kt, want = k[0, 0].double().t().contiguous(), torch.zeros(S, dtype=torch.float64, device=DEV)
+    for r in range(S - W, S, 2048):
+        lg = q[0, 0, r:r + 2048].double() @ kt * 0.125
+        later = torch.arange(S, device=DEV)[None] > torch.arange(r, r + lg.shape[0], device=DEV)[:, None]
+        want += torch.softmax(lg.masked_fill_(later, float("-inf")), dim=-1).sum(dim=0)
+    if pool > 1:
+        want = torch.nn.functional.avg_pool1d(want[None], pool, 1, pool // 2)[0]
+    assert torch.allclose(got[0, 0].double(), want, rtol=2.0 ** -21 + 2.0 ** -23, atol=0.0)
 
 
 def test_snapkv_scores_and_keep_llama8b_8k_layer():
@@ -924,7 +959,7 @@ H2O_CASES = [
     (2, 8, 2, 200, 16, torch.float16),
     (1, 32, 8, 333, 64, torch.float16),
     (1, 8, 8, 97, 128, torch.bfloat16),
-    # windows of 1024 rows or more: importance over mirrored key pairs
+    # windows of 256 rows or more: the importance chains split over four waves
     (1, 4, 2, 1500, 64, torch.float16),
     (1, 2, 1, 2049, 32, torch.bfloat16),     # odd S: the middle key once
 ]
