@@ -21,7 +21,8 @@
 //   qmean   -> qf (fp64 [B][Hk][Wpad][D], rows >= W zeroed)
 //   logits  -> L (fp32 [B][Hk][W][S]) + row max (atomicMax on order keys)
 //              (both in the int8-digit form of hc_logits_i8.h for 2-byte keys
-//              of head dim 64 or 128 and groups of 2^n query heads)
+//              of head dim 64 or 128, groups of 2^n query heads and a scale that
+//              is no power of two)
 //   rowsum  -> l_w (uint64, 64-bit atomics)            [SNAPKV only]
 //   imp     -> pooled fp32 scores [B][Hk][S]
 #include "hc_common.h"
@@ -756,8 +757,13 @@ __global__ void head_mean_kernel(const float* __restrict__ x, int H, int S, floa
 // against 87).
 constexpr int64_t kDigitLineRows = 32768;
 
-// The int8 kernel's workgroups at their fewest chunks: five per CU.
-constexpr int kDigitTargetWg = 1280;
+// The int8 kernel's workgroups that the chip holds at once: four per CU, three
+// with 64 window rows or raw sums.  A launch of few chunks is one round of them:
+// in two, the second waits for the first one's slowest (6 rows of 1936 keys, 8 KV
+// heads of 64, window 32: 1488 workgroups of a chunk 25.6 us, 744 of two 22.6).
+static int64_t digit_slots(int mode, int rows) {
+  return 256 * (mode == HC_SCORE_SNAPKV && rows < 64 ? 4 : 3);
+}
 
 template <typename T>
 static void launch_logits_i8(int mode, int64_t B, int64_t Hk, int64_t S, int64_t ld, int64_t D, int64_t W,
@@ -766,7 +772,7 @@ static void launch_logits_i8(int mode, int64_t B, int64_t Hk, int64_t S, int64_t
                              const QDigitRow* qrow, double scal, float* logits, uint32_t* rmax, hipStream_t st) {
   const int rows = W > 32 ? 64 : (W > 16 ? 32 : 16);     // wpad is a multiple of each
   const int64_t nrb = cdiv(W, rows), wg1 = cdiv(S, (int64_t)kDigitChunk) * Hk * nrb * B;
-  const int cpw = (int)std::max<int64_t>(1, std::min<int64_t>(kLogitChunks, wg1 / kDigitTargetWg));
+  const int cpw = (int)std::min<int64_t>(kLogitChunks, cdiv(wg1, digit_slots(mode, rows)));
   const dim3 grid((unsigned)cdiv(S, (int64_t)kDigitChunk * cpw), (unsigned)(Hk * nrb), (unsigned)B);
   auto launch = [&](auto kern) {
     hipLaunchKernelGGL(kern, grid, dim3(256), 0, st, k, k_rows, k_sb, k_sh, k_ss, k_bytes, qf, qd, qrow, (int)Hk,
@@ -781,7 +787,7 @@ static void launch_logits_i8(int mode, int64_t B, int64_t Hk, int64_t S, int64_t
       else launch(logits_i8_kernel<T, M, DC, 4>);
     };
     if (mode == HC_SCORE_SNAPKV) by_rows(std::integral_constant<int, HC_SCORE_SNAPKV>{});
-    else by_rows(std::integral_constant<int, HC_SCORE_RAWSUM>{});
+    else if constexpr (DC == 128) by_rows(std::integral_constant<int, HC_SCORE_RAWSUM>{});   // (sqrt(64) is dyadic)
   };
   if (D == 128) pick(std::integral_constant<int, 128>{});
   else pick(std::integral_constant<int, 64>{});
@@ -806,7 +812,14 @@ static void launch_score(const ScoreLayout& lay, char* ws, int mode, int64_t B, 
   // whose size is not a power of two has means that no fixed point holds, so
   // most of its tiles would be redone in fp64.
   const int64_t G = Hq % Hk == 0 ? Hq / Hk : Hq;
-  const bool dig = sizeof(T) == 2 && (D == 64 || D == 128) && (G & (G - 1)) == 0;
+  // A logit scale that is a power of two (head dim 64's own) leaves the exact dot
+  // products, which have few bits, on the midpoint of two floats in about one
+  // logit of 64: nearly every tile would be open.  Logits at 8 KV heads of 64,
+  // fp64 form against digits (us): f16 4 x 16384 keys, window 64, 106, 124;
+  // bf16 97, 138; 6 x 1936, window 32, 18, 23.
+  int exp2 = 0;
+  const bool dyadic = frexp(fabs(scal), &exp2) == 0.5;
+  const bool dig = sizeof(T) == 2 && (D == 64 || D == 128) && (G & (G - 1)) == 0 && !dyadic;
   const uint32_t k_bytes = (uint32_t)(((S - 1) * k_ss + D) * (int64_t)sizeof(T));
   bool done = false;
   if constexpr (sizeof(T) == 2) {
