@@ -14,7 +14,9 @@
 // With delta the sum of these, a logit whose dot product -delta and +delta
 // round to one float is that float; a 16 x 16 tile with any other logit is
 // recomputed by the fp64 chain itself (chain_tiles): 0.7 to 0.8% of the tiles of
-// N(0,1) prompts, a count over 12000.
+// N(0,1) prompts, a count over 12000.  (Not under a scale that is a power of two:
+// the exact products then fall on midpoints of floats, and the host takes the
+// fp64 kernel.)
 //
 // Keys with bits below the window (f16 tiles of wide channels, a bf16 tile in
 // some hundred) take a fifth digit, four more products (KDigits::low).  What
